@@ -148,16 +148,10 @@ def kernel_bytes(kernel: str, w, args) -> float:
     if kernel == "fwd_e":
         core = 24 if two_d else 48      # H read, E read+write, ca, ce_curl (+ce_rhs in 3D)
         return cells * (core + comps * hist_b * frames / w.sampling_interval) + 8 * pe
-    if kernel in ("adj_weights_e", "adj_weights_h"):
-        # lambda (3) + curl coefficient read, six channel weights written, lambda psi read+write
-        return cells * 40 + 8 * (pe if kernel == "adj_weights_e" else ph)
     if kernel == "adj_e":
-        return cells * 48               # six channel weights read, lambda_H read+write
+        return cells * 40 + 8 * pe      # lambda_E, ccurl read, lambda_H read+write, lambda psi_E read+write
     if kernel == "adj_h":
-        return cells * 52               # six channel weights read, lambda_E read+write, ca
-    if kernel == "adj_e_w":
-        # gather_e, then the H-side weights: W_E read, lambda_H read+write, hcurl, W_H written
-        return cells * 76 + 8 * ph
+        return cells * 44 + 8 * ph      # lambda_H, hcurl, ca read, lambda_E read+write, lambda psi_H read+write
     if kernel == "material_gradient":
         acc = 8 if args.accumulator == "float64" else 4
         return cells * (2 * comps * hist_b + 12) + ext * 2 * 2 * acc
@@ -175,11 +169,6 @@ def kernel_bytes(kernel: str, w, args) -> float:
 MEASURED_TRAFFIC = {
     ("c2", "tm_step_adj", "float32", "float64", 20): (121.9e6, "profiles/c2_fwi_2d_o4_tm_step_kernels.md"),
     ("c2", "tm_step_fwd", "float32", "float64", 20): (90.4e6, "profiles/c2_fwi_2d_o4_tm_step_kernels.md"),
-    ("c3", "fwd_e", "float32", "float64", 1): (1656.4e6, "profiles/c3_layered_3d_o4_kernels.md"),
-    ("c3", "fwd_h", "float32", "float64", 1): (1383.7e6, "profiles/c3_layered_3d_o4_kernels.md"),
-    ("c3", "adj_e_w", "float32", "float64", 1): (2204.0e6, "profiles/c3_layered_3d_o4_kernels.md"),
-    ("c3", "adj_h", "float32", "float64", 1): (1520.4e6, "profiles/c3_layered_3d_o4_kernels.md"),
-    ("c3", "adj_weights_e", "float32", "float64", 1): (1058.7e6, "profiles/c3_layered_3d_o4_kernels.md"),
 }
 
 

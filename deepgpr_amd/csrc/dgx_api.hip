@@ -535,6 +535,21 @@ bool xmarch3d()
     return v && std::strcmp(v, "xmarch") == 0;
 }
 
+// Solves of order 2 and 4 with a large enough interior run the row sweeps
+// (dgx_rows.hip); DEEPGPR_AMD_3D_SWEEP=cells keeps the one-thread-per-cell
+// sweeps, which order 8, smaller 3D grids and the general 2D path take (same
+// bits). So do the switches of those sweeps. Read at every solve.
+bool row_sweeps(const Grid& g, int order)
+{
+    const char* v = std::getenv("DEEPGPR_AMD_3D_SWEEP");
+    if (v && (std::strcmp(v, "cells") == 0 || std::strcmp(v, "xmarch") == 0)) return false;
+    v = std::getenv("DEEPGPR_AMD_3D_BOX");
+    if (v && std::strcmp(v, "off") == 0) return false;
+    v = std::getenv("DEEPGPR_AMD_3D_INTERLEAVE");
+    if (v && std::strcmp(v, "off") == 0) return false;
+    return adj3d_fused() && row_sweep_applies(g.N, g.pml, order);
+}
+
 // Static rule for the tile rows of a single fused TM solve. Small solves
 // leave most of the GPU idle and their time is the chain of one workgroup,
 // which shorter tiles cut: kTmBITiny when its kTmBITiny-row tiles over all
@@ -937,6 +952,52 @@ void receiver_groups(const std::vector<int>& rloc, int nshot, int nrx, long long
     }
 }
 
+// Receivers of the row sweeps by owning workgroup (of all shots), in receiver
+// order within one.
+void row_receiver_lists(const Grid& g, const RowMap& rm, const std::vector<int>& rloc, int nrx, std::vector<int>& off,
+                        std::vector<int2>& ent)
+{
+    const long long per = rm.total;
+    std::vector<std::pair<long long, int2>> tmp;
+    for (int s = 0; s < g.nshot; ++s)
+        for (int r = 0; r < nrx; ++r) {
+            const int* L = &rloc[((size_t)s * nrx + r) * 3];
+            tmp.push_back({row_block_of(rm, L[0], L[1]) + per * s,
+                           make_int2((int)(L[0] * g.st0 + (long long)L[1] * g.N[2] + L[2]), r)});
+        }
+    std::stable_sort(tmp.begin(), tmp.end(), [](const std::pair<long long, int2>& x,
+                                                const std::pair<long long, int2>& y) { return x.first < y.first; });
+    off.assign((size_t)(per * g.nshot) + 1, 0);
+    ent.clear();
+    for (const auto& e : tmp) {
+        off[(size_t)e.first + 1] += 1;
+        ent.push_back(e.second);
+    }
+    for (size_t k = 1; k < off.size(); ++k) off[k] += off[k - 1];
+}
+
+// The receiver groups (receiver_groups) of the row sweeps by owning workgroup.
+void row_receiver_groups(const Grid& g, const RowMap& rm, const std::vector<int>& goff, const std::vector<int>& gshot,
+                         const std::vector<long long>& gcell, std::vector<int>& off, std::vector<int4>& grp)
+{
+    const long long per = rm.total;
+    std::vector<std::pair<long long, int4>> tmp;
+    for (size_t q = 0; q < gshot.size(); ++q) {
+        const int i = (int)(gcell[q] / g.st0), j = (int)(gcell[q] % g.st0) / g.N[2];
+        tmp.push_back({row_block_of(rm, i, j) + per * gshot[q],
+                       make_int4((int)gcell[q], goff[q], goff[q + 1] - goff[q], 0)});
+    }
+    std::stable_sort(tmp.begin(), tmp.end(), [](const std::pair<long long, int4>& x,
+                                                const std::pair<long long, int4>& y) { return x.first < y.first; });
+    off.assign((size_t)(per * g.nshot) + 1, 0);
+    grp.clear();
+    for (const auto& e : tmp) {
+        off[(size_t)e.first + 1] += 1;
+        grp.push_back(e.second);
+    }
+    for (size_t k = 1; k < off.size(); ++k) off[k] += off[k - 1];
+}
+
 // Device copy of a host-built list (nothing to do for an empty one).
 template <typename T>
 bool upload(DevBuf& d, const std::vector<T>& v, hipStream_t st)
@@ -1000,6 +1061,8 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
     const bool fused = tm && tm2d_fused();
     const bool xm = !fixed && !tm && xmarch3d();
     const XmTiles xt = xm_tiles(g, pl.order);
+    const bool rows = !fixed && !tm && !xm && row_sweeps(g, pl.order);
+    const RowMap rm = rows ? row_map(g, pl.order) : RowMap{};
     if (fixed && pl.kind == kInt8 && pl.history) {
         set_error("dgx_forward_noalloc: INT8 histories need a scratch frame; use dgx_forward");
         return -1;
@@ -1007,7 +1070,8 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
     const Tm2dGrid tg = tm_grid_of(pl, fused ? tm2d_tile_rows(pl, P, stream) : kTmBI);
     const int tm_tiles = (g.N[0] * g.N[1] + 255) / 256;
     long long nblocks = tm ? (long long)tm_tiles * g.nshot
-                           : (xm ? (long long)xt.nty * xt.ntz * g.nshot : sweep.blocks);
+                           : (xm ? (long long)xt.nty * xt.ntz * g.nshot
+                                 : (rows ? (long long)rm.total * g.nshot : sweep.blocks));
     std::vector<int> boff((size_t)nblocks + 1, 0);
     std::vector<int2> ents;
     if (inject && fused) {
@@ -1026,7 +1090,8 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
                 long long m = (long long)L[0] * g.st0 + (long long)L[1] * g.N[2] + L[2];
                 // x-marching sweeps: one list per (shot, tile), in plane order
                 long long blk = xm ? ((long long)s * xt.nty * xt.ntz + xm_tile_of(xt, L[1], L[2])) * g.N[0] + L[0]
-                                   : cell_block(sweep, g, L[0], L[1], L[2], s);
+                                   : (rows ? row_block_of(rm, L[0], L[1]) + (long long)rm.total * s
+                                           : cell_block(sweep, g, L[0], L[1], L[2], s));
                 if (blk < 0 && !tm) {
                     set_error("forward: source cell outside the cell sweep");
                     return -1;
@@ -1103,6 +1168,25 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
         trx.count = (int)rent.size();
     }
 
+    // --- receivers of the row sweeps: grouped by owning workgroup ------------
+    RowReceivers rrx{};
+    if (rows && P->nreceiver > 0) {
+        std::vector<int> roff;
+        std::vector<int2> rent;
+        row_receiver_lists(g, rm, hrloc, P->nreceiver, roff, rent);
+        if (!upload(d_roff, roff, stream) || !upload(d_rent, rent, stream)) {
+            set_error("forward: out of device memory for receiver lists");
+            return -1;
+        }
+        rrx.off = (const int*)d_roff.p;
+        rrx.ent = (const int2*)d_rent.p;
+        rrx.out = P->receiver_data;
+        rrx.nrx = P->nreceiver;
+        rrx.nt = nt;
+        rrx.comp = rcomp;
+        rrx.count = (int)rent.size();
+    }
+
     // --- history buffers -----------------------------------------------------
     const bool int8 = pl.kind == kInt8;
     if (pl.history && (!P->E_saved || ((pl.store_r || pl.e_only) && !P->R_saved))) {
@@ -1138,6 +1222,16 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
     a.has_cpml = pl.has_cpml;
     a.src = src;
     const size_t eb = elem_bytes(pl.kind);
+    DevBuf d_tab;
+    if (rows && pl.has_cpml) {
+        if (!d_tab.alloc((size_t)8 * (g.N[0] + g.N[1] + g.N[2]) * sizeof(float))) {
+            set_error("forward: out of device memory for the CPML tables");
+            return -1;
+        }
+        launch_profile_tables(g, pl.cpe, pl.cph, (float*)d_tab.p, stream);
+        a.tab_e = (const float*)d_tab.p;
+        a.tab_h = a.tab_e + 4LL * (g.N[0] + g.N[1] + g.N[2]);
+    }
     DevBuf d_kc;  // grid, CPML and coefficients of the x-marching sweeps
     if (xm) {
         const XmConst kc = xm_const(g, pl.cpe, pl.cph, co[0], co[1], co[2], co[4], co[5]);
@@ -1255,6 +1349,9 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
         } else if (xm) {
             TIMED(tmr, kKXmFwdH, launch_xm_fwd_h(pl.order, g, xt, kcp, a, stream));
             TIMED(tmr, kKXmFwdE, launch_xm_fwd_e(pl.order, g, xt, kcp, a, stream));
+        } else if (rows) {
+            TIMED(tmr, kKFwdH, launch_row_fwd_h(pl.order, g, rm, a, stream));
+            TIMED(tmr, kKFwdE, launch_row_fwd_e(pl.order, g, rm, a, rrx, stream));
         } else {
             TIMED(tmr, kKFwdH, launch_fwd_h(pl.order, g, a, stream));
             TIMED(tmr, kKFwdE, launch_fwd_e(pl.order, g, a, stream));
@@ -1263,7 +1360,7 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
             TIMED(tmr, kKQuant,
                   launch_quant_int8(g, a.Ec, (const float*)d_rscratch.p, pl.snap,
                                     int8_writer(pl, P->R_saved, pl.nt_saved, ts), stream));
-        if (P->nreceiver > 0 && !fused_rx) {
+        if (P->nreceiver > 0 && !fused_rx && !rows) {
             if (tm && rcomp == 2)
                 TIMED(tmr, kKSample,
                       launch_sample(g, tms.f.Ez, P->receiver_location, P->receiver_data, P->nreceiver, nt, it,
@@ -1425,7 +1522,29 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
 
     const bool xm = !tm && xmarch3d();
     const XmTiles xt = xm_tiles(g, pl.order);
-    const bool fuse3 = !tm && !xm && adj3d_fused();
+    const bool rows = !tm && !xm && row_sweeps(g, pl.order);
+    const RowMap rm = rows ? row_map(g, pl.order) : RowMap{};
+    const bool fuse3 = !tm && !xm && !rows && adj3d_fused();
+
+    // row sweeps: the receiver groups by owning workgroup
+    DevBuf d_ooff, d_ogrp;
+    RowAdjReceivers rax{};
+    if (rows && adj_rx && !gshot.empty()) {
+        std::vector<int> ooff;
+        std::vector<int4> ogrp;
+        row_receiver_groups(g, rm, goff, gshot, gcell, ooff, ogrp);
+        if (!upload(d_ooff, ooff, stream) || !upload(d_ogrp, ogrp, stream)) {
+            set_error("backward: out of device memory for receiver lists");
+            return -1;
+        }
+        rax.off = (const int*)d_ooff.p;
+        rax.grp = (const int4*)d_ogrp.p;
+        rax.member = rg.member;
+        rax.dgrad = P->data_grad;
+        rax.nrx = P->nreceiver;
+        rax.nt = nt;
+        rax.comp = P->receiver_component;
+    }
 
     // fused 2D TM kernels: the groups again, listed for every (tile, shot)
     // whose staged region (tile plus halo) holds the cell
@@ -1496,7 +1615,7 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
             tw.wh[f] = p;
             p += across * g.pml[f];
         }
-    } else if (!tm && !xm) {
+    } else if (!tm && !xm && !rows) {
         // six channel-weight arrays: shared by the E and H halves of the
         // adjoint, or one set per half when the gathers write the next weights
         const long long wlen = (fuse3 ? 12LL : 6LL) * g.nshot * g.cells;
@@ -1505,6 +1624,37 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
             return -1;
         }
     }
+
+    // row sweeps: second copies of the lambda psi arrays of the x and y faces; a
+    // half step reads its neighbours' old ones while it writes its own (those
+    // of the z faces are read at their own cells alone)
+    DevBuf d_psi;
+    Cpml psi_set[2][2] = {{pl.cpe, pl.cph}, {pl.cpe, pl.cph}};  // [copy][E, H]
+    CopySpans psi_copy{};
+    if (rows && pl.has_cpml && nt > 0) {
+        long long tot = 0;
+        for (int eh = 0; eh < 2; ++eh)
+            for (int f = 0; f < 4; ++f)
+                for (int w = 0; w < 2; ++w) tot += psi_elems(g, eh == 0, f, w);
+        if (!d_psi.alloc((size_t)tot * sizeof(float))) {
+            set_error("backward: out of device memory for the CPML auxiliaries (%lld bytes)", tot * 4);
+            return -1;
+        }
+        float* p = (float*)d_psi.p;
+        for (int eh = 0; eh < 2; ++eh)
+            for (int f = 0; f < 4; ++f)
+                for (int w = 0; w < 2; ++w) {
+                    const long long n = psi_elems(g, eh == 0, f, w);
+                    if (n <= 0) continue;
+                    psi_copy.from[psi_copy.count] = psi_set[0][eh].psi[f][w];
+                    psi_copy.to[psi_copy.count] = p;
+                    psi_copy.n[psi_copy.count++] = n;
+                    psi_set[1][eh].psi[f][w] = p;
+                    p += n;
+                }
+        launch_copy_spans(psi_copy, stream);  // elements that no cell advances stay equal in both
+    }
+    int psi_at = 0;
 
     // FP64 accumulators of the time-summed material gradients
     const long long ngrad = (long long)(g.N[0] - 1) * (g.N[1] - 1) * (g.N[2] - 1);
@@ -1539,6 +1689,16 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
     a.cpe = pl.cpe;
     a.cph = pl.cph;
     a.has_cpml = pl.has_cpml;
+    DevBuf d_tab;
+    if (rows && pl.has_cpml) {
+        if (!d_tab.alloc((size_t)8 * (g.N[0] + g.N[1] + g.N[2]) * sizeof(float))) {
+            set_error("backward: out of device memory for the CPML tables");
+            return -1;
+        }
+        launch_profile_tables(g, pl.cpe, pl.cph, (float*)d_tab.p, stream);
+        a.tab_e = (const float*)d_tab.p;
+        a.tab_h = a.tab_e + 4LL * (g.N[0] + g.N[1] + g.N[2]);
+    }
     DevBuf d_kc;  // grid, CPML and coefficients of the x-marching sweeps
     if (xm) {
         const XmConst kc = xm_const(g, pl.cpe, pl.cph, co[0], co[1], co[2], co[4], co[5]);
@@ -1596,7 +1756,7 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
             tms.flip();
             continue;
         }
-        if (adj_rx)
+        if (adj_rx && (!rows || it == nt - 1))  // the row sweeps add the later ones themselves
             TIMED(tmr, kKAdjRx, launch_adj_receivers(gc, rg, lam_rx, P->data_grad, P->nreceiver, nt, it, stream));
         if (want_src)
             TIMED(tmr, kKAdjSrc,
@@ -1618,6 +1778,19 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
         } else if (xm) {
             TIMED(tmr, kKXmAdjE, launch_xm_adj(pl.order, true, g, xt, kcp, a, it != nt - 1, stream));
             TIMED(tmr, kKXmAdjH, launch_xm_adj(pl.order, false, g, xt, kcp, a, false, stream));
+        } else if (rows) {
+            const Cpml* from = psi_set[psi_at];
+            const Cpml* to = psi_set[psi_at ^ 1];
+            PsiOut oe{}, oh{};
+            std::memcpy(oe.psi, to[0].psi, sizeof(oe.psi));
+            std::memcpy(oh.psi, to[1].psi, sizeof(oh.psi));
+            a.cpe = from[0];
+            a.cph = from[1];
+            rax.it = it - 1;
+            rax.count = it > 0 ? rg.ngroups : 0;
+            TIMED(tmr, kKAdjE, launch_row_adj(pl.order, true, g, rm, a, oe, rax, stream));
+            TIMED(tmr, kKAdjH, launch_row_adj(pl.order, false, g, rm, a, oh, rax, stream));
+            psi_at ^= 1;
         } else if (fuse3) {
             float* We = (float*)d_w.p;
             float* Wh = We + 6LL * g.nshot * g.cells;
@@ -1631,6 +1804,14 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
             TIMED(tmr, kKAdjWeightsH, launch_adj_weights(pl.order, false, g, a, W, stream));
             TIMED(tmr, kKAdjH, launch_adj_gather_h(pl.order, g, a, W, stream));
         }
+    }
+    if (psi_at) {  // the caller's arrays hold the last but one
+        CopySpans back = psi_copy;
+        for (int q = 0; q < back.count; ++q) {
+            back.from[q] = psi_copy.to[q];
+            back.to[q] = const_cast<float*>(psi_copy.from[q]);
+        }
+        launch_copy_spans(back, stream);
     }
     if (xm && nt > 0) TIMED(tmr, kKXmPsiH, launch_xm_psi_h_final(g, kcp, a, stream));
     if (tm && tms.unpack(P, stream)) {
@@ -2307,6 +2488,9 @@ DGX_API long long dgx_scratch_bytes(const dgx_solve* solve, int backward)
         if (xmarch3d()) {
             const XmTiles xt = xm_tiles(g, pl.order);
             bytes += ((long long)xt.nty * xt.ntz * g.nshot + 1) * 4;
+        } else if (row_sweeps(g, pl.order)) {
+            // source and receiver lists
+            bytes += 2 * ((long long)row_map(g, pl.order).total * g.nshot + 1) * 4;
         } else {
             bytes += (cell_sweep(g, pl.order).blocks + 1) * 4;
         }
@@ -2318,7 +2502,7 @@ DGX_API long long dgx_scratch_bytes(const dgx_solve* solve, int backward)
         // adjoint channel weights of the general (non-2D-TM) path
         const bool tm_shape = (solve->storage_type & kFlagTm2d) && g.N[2] == 2 && solve->source_component == 2 &&
                               pl.kind != kInt8;
-        if (!tm_shape && !xmarch3d()) bytes += (adj3d_fused() ? 48LL : 24LL) * g.nshot * g.cells;
+        if (!tm_shape && !xmarch3d() && !row_sweeps(g, pl.order)) bytes += (adj3d_fused() ? 48LL : 24LL) * g.nshot * g.cells;
     }
     return bytes;
 }

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "dgx_device.h"
+#include "dgx_rows.h"
 
 namespace dgx {
 
@@ -78,6 +79,7 @@ struct StepArgs {
     CF3 Ec, Hc;
     Cpml cpe, cph;
     int has_cpml;
+    const float *tab_e, *tab_h;  // CPML profiles by cell (row sweeps)
     SourceBlocks src;
     HistWrite hist;
 };
@@ -88,6 +90,7 @@ struct AdjArgs {
     CF3 lEc, lHc;
     Cpml cpe, cph;  // lambda psi arrays + profiles
     int has_cpml;
+    const float *tab_e, *tab_h;  // CPML profiles by cell (row sweeps)
 };
 
 // 2D Ez-TM fast path: compact (nshot, NX, NY) state, y fastest.
@@ -295,6 +298,48 @@ void launch_adj_gather_e(int order, const Grid& g, const AdjArgs& a, const float
 void launch_adj_gather_h(int order, const Grid& g, const AdjArgs& a, const float* W, hipStream_t st);
 // the E-side gather fused with the H-side weights: W_E -> lambda_H -> W_H
 void launch_adj_gather_e_w(int order, const Grid& g, const AdjArgs& a, const float* We, float* Wh, hipStream_t st);
+
+// Row sweeps of the 3D solver (dgx_rows.hip; block map in dgx_rows.h).
+// Receivers read by the electric sweep: entries (cell, receiver) of workgroup
+// b (of all shots) are ent[off[b] .. off[b + 1]).
+struct RowReceivers {
+    const int* off;
+    const int2* ent;
+    float* out;  // (nshot, nt, nrx)
+    int nrx, nt, comp, count;
+};
+// Receiver groups added by the adjoint's magnetic half step to lambda_E for
+// step `it`: grp = (cell, first member, members, 0), by workgroup.
+struct RowAdjReceivers {
+    const int* off;
+    const int4* grp;
+    const int* member;
+    const float* dgrad;  // (nshot, nt, nrx)
+    int nrx, nt, it, comp, count;
+};
+// Where a half step writes the advanced CPML auxiliaries (it reads its
+// neighbours' old ones).
+struct PsiOut {
+    float* psi[6][2];
+};
+// Arrays copied in one launch.
+constexpr int kMaxCopies = 24;
+struct CopySpans {
+    const float* from[kMaxCopies];
+    float* to[kMaxCopies];
+    long long n[kMaxCopies];
+    int count;
+};
+RowMap row_map(const Grid& g, int order);
+void launch_row_fwd_h(int order, const Grid& g, const RowMap& rm, const StepArgs& a, hipStream_t st);
+void launch_row_fwd_e(int order, const Grid& g, const RowMap& rm, const StepArgs& a, const RowReceivers& rx,
+                      hipStream_t st);
+void launch_row_adj(int order, bool electric, const Grid& g, const RowMap& rm, const AdjArgs& a, const PsiOut& po,
+                    const RowAdjReceivers& rx, hipStream_t st);
+// The CPML profiles by cell: electric, then magnetic; of each axis RA - 1, RB, RE
+// and RF, N[axis] cells each (zero outside the faces).
+void launch_profile_tables(const Grid& g, const Cpml& cpe, const Cpml& cph, float* tab, hipStream_t st);
+void launch_copy_spans(const CopySpans& sp, hipStream_t st);
 
 // x-marching 3D sweeps (dgx_xmarch.hip): a workgroup owns a (y, z) tile of
 // `ty` rows (one wavefront each) x 64 cells of one shot and walks `xc`

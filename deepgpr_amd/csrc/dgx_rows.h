@@ -1,0 +1,194 @@
+// Block -> cell mapping of the row sweeps (dgx_rows.hip), shared by the
+// kernels, the host launch code and a host-only test.
+//
+// A workgroup owns some consecutive rows of one x-plane of one shot, over
+// their whole z extent; its threads take the rows one after another in groups
+// of consecutive cells. The last group of a row is moved back to end with the
+// row: its first cells belong to the group before it. There are two kinds of
+// workgroups: plain ones, whose rows lie in the plain ranges of x and y, with
+// groups of V cells, and edge ones with groups of V / 2 cells (their code holds
+// more values a cell).
+#pragma once
+
+#include "dgx_sweep.h"
+
+namespace dgx {
+
+struct RowKind {
+    int gpr;   // groups of a row
+    int rb;    // rows of a workgroup
+    Div div;   // / gpr
+};
+
+struct RowMap {
+    RowKind plain, edge;
+    int V;               // cells of a plain group
+    int threads;         // threads of a workgroup (a multiple of 64)
+    int lds;             // floats of one row buffer of a workgroup
+    int n0, n1, n2;      // the grid
+    int xlo, xhi, ylo, yhi, zlo, zhi;  // plain ranges (inclusive)
+    int ne, nm;          // edge and plain workgroups of an inner plane (i in [xlo, xhi])
+    int nylo;            // of the ne, those of rows below ylo
+    int bo, bi;          // workgroups of an outer / inner plane, padded to multiples of 8
+    int to, ti;          // of all outer / inner planes
+    int ratio;           // bundles of 8 inner workgroups after one of outer ones
+    int total;           // workgroups of a shot
+    Div div_bo, div_bi, div_group;  // / bo, / bi, / (8 (1 + ratio))
+};
+
+// Plain range along one axis of n cells with CPML widths plo and phi: cells
+// whose stencils, and the transposed stencils of the adjoint, are full-width,
+// see no CPML term of this axis and read only updated cells.
+DGX_HD void row_plain_range(int n, int plo, int phi, int R, int& lo, int& hi)
+{
+    lo = 2 * R - 1;
+    if (plo > 0 && plo + R > lo) lo = plo + R;
+    hi = n - 2 * R;
+    if (n - 2 - R < hi) hi = n - 2 - R;
+    if (phi > 0 && n - 2 - phi - R < hi) hi = n - 2 - phi - R;
+}
+
+// The row sweeps take solves of order 2 and 4 on grids with a plain interior
+// that is worth it: at least 65536 cells plain for every order, in rows of at
+// least 32 of them and at most 1024 cells (a row fits a workgroup of 512
+// threads), and a field array of a shot below 4 GiB (32-bit offsets). An
+// order-8 cell has so many taps that its values fill the registers of a
+// thread (us per step on an MI355X, row sweeps / one thread per cell: forward
+// 118 / 100, adjoint 199 / 152 on 138 x 120 x 152 fields).
+inline bool row_sweep_applies(const int N[3], const int pml[6], int order)
+{
+    if (order > 4) return false;
+    long long cells = 1;
+    for (int a = 0; a < 3; ++a) {
+        int lo, hi;
+        row_plain_range(N[a], pml[2 * a], pml[2 * a + 1], 4, lo, hi);
+        if (hi < lo) return false;
+        if (a == 2 && hi - lo + 1 < 32) return false;
+        cells *= hi - lo + 1;
+    }
+    return cells >= 65536 && N[2] <= 1024 && 1LL * N[0] * N[1] * N[2] < (1LL << 30);
+}
+
+// Rows of a workgroup: the count within max_threads that leaves the fewest
+// lanes idle, the larger of nearly equal ones.
+inline RowKind make_row_kind(int n2, int V, int max_threads)
+{
+    RowKind k{};
+    k.gpr = (n2 + V - 1) / V;
+    k.div = make_div((unsigned)k.gpr);
+    double best = 0.0;
+    for (int rb = 1; rb <= 16; ++rb) {
+        const int t = (rb * k.gpr + 63) / 64 * 64;
+        if (rb > 1 && t > max_threads) break;
+        const double use = (double)rb * k.gpr / t;
+        if (use > best - 0.02) {
+            best = use > best ? use : best;
+            k.rb = rb;
+        }
+    }
+    return k;
+}
+
+inline RowMap make_row_map(const int N[3], const int pml[6], int R, int V, int max_threads)
+{
+    RowMap m{};
+    m.V = V;
+    m.n0 = N[0];
+    m.n1 = N[1];
+    m.n2 = N[2];
+    row_plain_range(N[0], pml[0], pml[1], R, m.xlo, m.xhi);
+    row_plain_range(N[1], pml[2], pml[3], R, m.ylo, m.yhi);
+    row_plain_range(N[2], pml[4], pml[5], R, m.zlo, m.zhi);
+    m.plain = make_row_kind(N[2], V, max_threads);
+    m.edge = make_row_kind(N[2], V / 2, max_threads);
+    const int tp = m.plain.rb * m.plain.gpr, te = m.edge.rb * m.edge.gpr;
+    m.threads = ((tp > te ? tp : te) + 63) / 64 * 64;
+    const int lp = tp * V, le = te * (V / 2);
+    m.lds = ((lp > le ? lp : le) + 3) / 4 * 4;
+    auto blocks = [](int rows, int rb) { return (rows + rb - 1) / rb; };
+    auto pad8 = [](int n) { return (n + 7) / 8 * 8; };
+    m.nylo = blocks(m.ylo, m.edge.rb);
+    m.ne = m.nylo + blocks(m.n1 - 1 - m.yhi, m.edge.rb);
+    m.nm = blocks(m.yhi - m.ylo + 1, m.plain.rb);
+    m.bi = pad8(m.ne + m.nm);
+    m.bo = pad8(blocks(m.n1, m.edge.rb));
+    m.ti = m.bi * (m.xhi - m.xlo + 1);
+    m.to = m.bo * (m.n0 - (m.xhi - m.xlo + 1));
+    m.ratio = (m.ti + m.to / 2) / m.to;
+    if (m.ratio < 1) m.ratio = 1;
+    const int go = m.to / 8, gi = (m.ti / 8 + m.ratio - 1) / m.ratio;
+    m.total = (go > gi ? go : gi) * 8 * (1 + m.ratio);
+    m.div_bo = make_div((unsigned)m.bo);
+    m.div_bi = make_div((unsigned)m.bi);
+    m.div_group = make_div((unsigned)(8 * (1 + m.ratio)));
+    return m;
+}
+
+// Workgroup b of a shot: its kind (1 plain, 0 edge, -1 none), plane, first row
+// and row count. The outer planes' workgroups (CPML along x) are spread among
+// the others, so that their longer chains run beside them. Workgroup b runs on
+// XCD b mod 8, and so does the same row block of the next plane (bundles of 8,
+// bo and bi multiples of 8): x-neighbours meet in one L2.
+DGX_HD int row_block(const RowMap& m, int b, int& i, int& j0, int& nj)
+{
+    const int span = 8 * (1 + m.ratio);
+    const int g = (int)div_q((unsigned)b, m.div_group), r = b - g * span;
+    if (r < 8) {
+        const int o = g * 8 + r;
+        if (o >= m.to) return -1;
+        const int pl = (int)div_q((unsigned)o, m.div_bo);
+        i = pl < m.xlo ? pl : pl + (m.xhi - m.xlo + 1);
+        j0 = (o - pl * m.bo) * m.edge.rb;
+        nj = m.n1 - j0 < m.edge.rb ? m.n1 - j0 : m.edge.rb;
+        return nj > 0 ? 0 : -1;
+    }
+    const int o = g * 8 * m.ratio + r - 8;
+    if (o >= m.ti) return -1;
+    const int pl = (int)div_q((unsigned)o, m.div_bi);
+    const int p = o - pl * m.bi;
+    i = m.xlo + pl;
+    if (p < m.ne) {
+        const bool low = p < m.nylo;
+        j0 = low ? p * m.edge.rb : m.yhi + 1 + (p - m.nylo) * m.edge.rb;
+        const int end = low ? m.ylo : m.n1;
+        nj = end - j0 < m.edge.rb ? end - j0 : m.edge.rb;
+        return 0;
+    }
+    j0 = m.ylo + (p - m.ne) * m.plain.rb;
+    nj = m.yhi + 1 - j0 < m.plain.rb ? m.yhi + 1 - j0 : m.plain.rb;
+    return nj > 0 ? 1 : -1;
+}
+
+// Thread t of a workgroup of nj rows: its row, the first cell k of its group of
+// V cells and how many of the group's first cells belong to the group before
+// it; false for an idle thread (row, k and dup are then those of a valid one).
+DGX_HD bool row_thread(const RowMap& m, const RowKind& kd, int V, int t, int nj, int& row, int& k, int& dup)
+{
+    row = (int)div_q((unsigned)t, kd.div);
+    k = (t - row * kd.gpr) * V;
+    dup = 0;
+    if (k > m.n2 - V) {
+        dup = k - (m.n2 - V);
+        k = m.n2 - V;
+    }
+    if (row < nj) return true;
+    row = 0;
+    return false;
+}
+
+// Workgroup of a shot that owns row (i, j).
+inline int row_block_of(const RowMap& m, int i, int j)
+{
+    if (i < m.xlo || i > m.xhi) {
+        const int pl = i < m.xlo ? i : i - (m.xhi - m.xlo + 1);
+        const int o = pl * m.bo + j / m.edge.rb;
+        return o / 8 * 8 * (1 + m.ratio) + o % 8;
+    }
+    const int p = j < m.ylo ? j / m.edge.rb
+                            : (j > m.yhi ? m.nylo + (j - m.yhi - 1) / m.edge.rb : m.ne + (j - m.ylo) / m.plain.rb);
+    const int o = (i - m.xlo) * m.bi + p;
+    const int g = o / (8 * m.ratio);
+    return g * 8 * (1 + m.ratio) + 8 + o - g * 8 * m.ratio;
+}
+
+}  // namespace dgx

@@ -23,9 +23,11 @@ MEMORY_SAFETY_MARGIN = 1.20
 
 
 def _adjoint_weight_cells(nz: int) -> bool:
-    # the one-thread-per-cell 3D adjoint keeps six FP32 channel weights per
-    # cell and shot for each half step; the x-marching sweeps form them on
-    # the fly, and the 2D Ez-TM kernels recompute them on a halo
+    # the one-thread-per-cell 3D adjoint (order 8, small grids) keeps six FP32
+    # channel weights per cell and shot for each half step; the row sweeps of
+    # orders 2 and 4 and the x-marching sweeps form them on the fly, and the 2D
+    # Ez-TM kernels recompute them on a halo. The order is not known here, so
+    # every 3D adjoint is priced with them.
     return nz > 1 and os.environ.get("DEEPGPR_AMD_3D_SWEEP") != "xmarch"
 
 
@@ -40,9 +42,9 @@ def estimate_compute_memory(*, device, nx: int, ny: int, nz: int, nt: int, nstep
     category plus peaks (the reference's keywords and result keys; nx, ny, nz
     are the extended grid with the CPML). The figures are this build's:
     histories stay in HBM (use_async_offload changes nothing and
-    effective_async_offload is False); a 3D adjoint keeps twelve FP32 channel
-    weights per cell and shot in library scratch (adjoint_stencil_weights;
-    2D models are priced for the Ez-TM kernels of the default Ez source,
+    effective_async_offload is False); a 3D adjoint is priced with the twelve FP32 channel
+    weights per cell and shot that order 8 and small grids keep in library
+    scratch (adjoint_stencil_weights; 2D models are priced for the Ez-TM kernels of the default Ez source,
     which keep none);
     FP64 accumulators (gradient_accumulator="float64", the default) add 16 B
     per model cell to material_gradients during the backward; no exact FP32
