@@ -120,7 +120,7 @@ const char* const kKernelNames[kKCount] = {
     "coefficients", "fwd_h", "fwd_e", "sample", "quant_int8", "save_frame", "adj_receivers",
     "adj_source", "material_gradient", "adj_pml_e", "adj_e", "adj_pml_h", "adj_h", "tm_step_fwd",
     "tm_step_adj", "tm_grad_reduce", "tm_src_reduce", "adj_weights_e", "adj_weights_h", "adj_e_w",
-    "xm_fwd_h", "xm_fwd_e", "xm_adj_e", "xm_adj_h", "xm_psi_h"};
+    "xm_fwd_h", "xm_fwd_e", "xm_adj_e", "xm_adj_h", "xm_psi_h", "tm_strip_fwd", "tm_strip_adj"};
 
 struct LaunchTimer {
     bool on;
@@ -513,6 +513,16 @@ bool tm2d_fused()
         return !(v && std::strcmp(v, "split") == 0);
     }();
     return fused;
+}
+
+// Several steps a launch (dgx_tm2d_strip.hip) where they apply;
+// DEEPGPR_AMD_TM2D_STRIPS=0 keeps one step a launch (same bits), and so do the
+// switches of the one-step kernels. Read on every call.
+bool tm2d_strips()
+{
+    const char* v = std::getenv("DEEPGPR_AMD_TM2D_STRIPS");
+    if (v && std::strcmp(v, "0") == 0) return false;
+    return !std::getenv("DEEPGPR_AMD_TM2D_TILE_ROWS");
 }
 
 // The 3D adjoint runs the E-side gather fused with the H-side weights;
@@ -920,6 +930,43 @@ void tm_receiver_groups(const Tm2dGrid& g, int order, const std::vector<int>& go
     for (size_t k = 1; k < off.size(); ++k) off[k] += off[k - 1];
 }
 
+// Entries of strip lists: grouped by (tile, shot), in input order within one.
+template <typename E>
+void strip_lists(std::vector<std::pair<long long, E>>& tmp, long long lists, std::vector<int>& off, std::vector<E>& ent)
+{
+    std::stable_sort(tmp.begin(), tmp.end(),
+                     [](const std::pair<long long, E>& a, const std::pair<long long, E>& b) { return a.first < b.first; });
+    off.assign((size_t)lists + 1, 0);
+    ent.clear();
+    for (const auto& e : tmp) {
+        off[(size_t)e.first + 1] += 1;
+        ent.push_back(e.second);
+    }
+    for (size_t k = 1; k < off.size(); ++k) off[k] += off[k - 1];
+}
+
+// Points of every shot (loc: nshot x n x 3) as (staged index, point) entries of
+// the tile that owns the cell or, with `margin`, of every tile that stages it.
+void strip_points(const StripMap& m, int nshot, const std::vector<int>& loc, int n, bool margin, std::vector<int>& off,
+                  std::vector<int2>& ent)
+{
+    std::vector<std::pair<long long, int2>> tmp;
+    for (int s = 0; s < nshot; ++s)
+        for (int k = 0; k < n; ++k) {
+            const int* L = &loc[((size_t)s * n + k) * 3];
+            int a0 = L[0] / m.orow, a1 = a0, b0 = L[1] / m.ocol, b1 = b0;
+            if (margin) {
+                strip_tiles(L[0], m.orow, m.sh.halo, m.sh.rows, m.nti, a0, a1);
+                strip_tiles(L[1], m.ocol, m.sh.halo, 64, m.ntj, b0, b1);
+            }
+            for (int a = a0; a <= a1; ++a)
+                for (int b = b0; b <= b1; ++b)
+                    tmp.push_back({a * m.ntj + b + (long long)m.tiles * s,
+                                   make_int2(strip_local(m, a, b, L[0], L[1]), k)});
+        }
+    strip_lists(tmp, (long long)m.tiles * nshot, off, ent);
+}
+
 // Receiver groups of one call: one per (shot, cell), members in receiver
 // order; cell = linear index with strides (st0, st1, 1).
 void receiver_groups(const std::vector<int>& rloc, int nshot, int nrx, long long st0, long long st1,
@@ -1067,14 +1114,20 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
         set_error("dgx_forward_noalloc: INT8 histories need a scratch frame; use dgx_forward");
         return -1;
     }
-    const Tm2dGrid tg = tm_grid_of(pl, fused ? tm2d_tile_rows(pl, P, stream) : kTmBI);
+    const Tm2dGrid tg0 = tm_grid_of(pl, kTmBI);
+    const bool strips = fused && tm2d_strips() && strip_applies(pl.order, tg0) &&
+                        (P->nreceiver <= 0 || P->receiver_component == 2);
+    const StripMap stm = strips ? strip_map(pl.order, tg0) : StripMap{};
+    const Tm2dGrid tg = !fused || strips ? tg0 : tm_grid_of(pl, tm2d_tile_rows(pl, P, stream));
     const int tm_tiles = (g.N[0] * g.N[1] + 255) / 256;
     long long nblocks = tm ? (long long)tm_tiles * g.nshot
                            : (xm ? (long long)xt.nty * xt.ntz * g.nshot
                                  : (rows ? (long long)rm.total * g.nshot : sweep.blocks));
     std::vector<int> boff((size_t)nblocks + 1, 0);
     std::vector<int2> ents;
-    if (inject && fused) {
+    if (inject && strips) {
+        strip_points(stm, g.nshot, hsloc, P->nsource, true, boff, ents);
+    } else if (inject && fused) {
         tm_source_lists(tg, hsloc, P->nsource, boff, ents);
     } else if (inject) {
         struct E4 {
@@ -1155,7 +1208,8 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
     if (fused_rx) {
         std::vector<int> roff;
         std::vector<int2> rent;
-        tm_receiver_lists(tg, hrloc, P->nreceiver, roff, rent);
+        if (strips) strip_points(stm, g.nshot, hrloc, P->nreceiver, false, roff, rent);
+        else tm_receiver_lists(tg, hrloc, P->nreceiver, roff, rent);
         if (!upload(d_roff, roff, stream) || !upload(d_rent, rent, stream)) {
             set_error("forward: out of device memory for receiver lists");
             return -1;
@@ -1254,7 +1308,7 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
     // remaining steps are launched one by one below.
     int it0 = 0;
     DevBuf d_step;
-    const bool graphed = fused && !pl.history && !tmr.on && tm2d_graphs() && nt >= 2 * kGraphSteps &&
+    const bool graphed = fused && !strips && !pl.history && !tmr.on && tm2d_graphs() && nt >= 2 * kGraphSteps &&
                          (P->nreceiver <= 0 || fused_rx);
     if (graphed) {
         // earlier launch errors are reported here: the fallback below clears
@@ -1306,6 +1360,25 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
             }
             (void)hipGetLastError();  // a failed capture falls back to launches one by one
         }
+    }
+    if (strips) {
+        StripHist sh{};
+        sh.on = pl.history;
+        sh.kind = pl.kind;
+        sh.mode = pl.comps == 3 ? 3 : 2;
+        sh.S = std::max(S, 1);
+        sh.e = P->E_saved;
+        sh.r = pl.store_r ? P->R_saved : nullptr;
+        sh.snap = pl.snap;
+        sh.cstride = pl.cstride;
+        sh.box = pl.box;
+        for (; it0 < nt; it0 += stm.sh.steps) {
+            TIMED(tmr, kKTmStripFwd,
+                  launch_tm_strip_fwd(pl.order, tms.g, tms.f, tms.pp, stm, a.src, trx, sh, it0,
+                                      std::min(stm.sh.steps, nt - it0), stream));
+            tms.flip();
+        }
+        it0 = nt;
     }
     for (int it = it0; it < nt; ++it) {
         const bool save = pl.history && (it % S) == 0;

@@ -434,6 +434,45 @@ __device__ __forceinline__ float gather_fwd_sel(WF wf, int c, int n)
 }
 
 // ---------------------------------------------------------------------------
+// Division by a grid spacing
+// ---------------------------------------------------------------------------
+// x[q] / d, correctly rounded, for n values at once: with y the correctly
+// rounded 1 / d, q = x y and r = x - q d (exact in one fused multiply-add),
+// q + r y rounds to the quotient (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990). That needs r not to
+// underflow and nothing to overflow, so values outside 2^-90 .. 2^90 (zeros
+// aside), infinities, NaN and spacings outside 2^-30 .. 2^30 take the division
+// proper.
+struct Spacing {
+    float d, y, big;
+};
+
+__host__ inline Spacing make_spacing(float d)
+{
+    return {d, 1.0f / d, d >= 0x1p-30f && d <= 0x1p30f ? 0.0f : 0x1p100f};
+}
+
+template <int N>
+__device__ __forceinline__ void div_all(const float (&x)[N], const Spacing& sp, float (&out)[N])
+{
+    const float d = sp.d, y = sp.y;
+    float big = sp.big;
+    unsigned small = ~0u;  // of the magnitudes' bits less one: a zero counts as the largest
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        const float t = x[q] * y;
+        out[q] = __builtin_fmaf(__builtin_fmaf(-t, d, x[q]), y, t);
+        // an unordered compare later takes a NaN; fmaxf would drop it
+        big = big + __builtin_fabsf(x[q]);
+        small = min(small, (__float_as_uint(x[q]) << 1) - 1u);
+    }
+    if (!(big < 0x1p90f) || small < (37u << 24)) {
+#pragma unroll
+        for (int q = 0; q < N; ++q) out[q] = x[q] / d;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Update masks (deepgpr_cpu.c:697-699, 913-915)
 // ---------------------------------------------------------------------------
 

@@ -3,6 +3,7 @@
 
 #include "dgx_device.h"
 #include "dgx_rows.h"
+#include "dgx_strip.h"
 
 namespace dgx {
 
@@ -254,6 +255,22 @@ void launch_tm_grad_reduce(const Tm2dGrid& g, const Box& b, const float* terms, 
                            void* geps, void* gsig, bool fp64, hipStream_t st);
 void launch_tm_src_reduce(const float* vals, float* gsrc, int nshot, int nsrc, int nt, hipStream_t st);
 
+// Strip kernels: several steps a launch (dgx_tm2d_strip.hip). Source and
+// receiver lists index staged cells (strip_local).
+struct StripHist {
+    int on;              // a history is kept
+    int kind, mode, S;
+    void *e, *r;         // E^n and R^n frames (null: not stored)
+    long long snap;      // elements of one frame of one component
+    long long cstride;   // elements between components
+    Box box;
+};
+bool strip_applies(int order, const Tm2dGrid& g);
+StripMap strip_map(int order, const Tm2dGrid& g);
+void launch_tm_strip_fwd(int order, const Tm2dGrid& g, const Tm2dFields& f, const TmPingPong& pp, const StripMap& sm,
+                         const SourceBlocks& src, const TmReceiversFwd& rx, const StripHist& hist, int it0, int nsub,
+                         hipStream_t st);
+
 void launch_tm_fwd_h(int order, const Tm2dGrid& g, const Tm2dFields& f, hipStream_t st);
 void launch_tm_fwd_e(int order, const Tm2dGrid& g, const Tm2dFields& f, const SourceBlocks& src,
                      const HistWrite& hw, hipStream_t st);
@@ -386,7 +403,8 @@ void launch_xm_psi_h_final(const Grid& g, const XmConst* kc, const AdjArgs& a, h
 enum KernelId : int {
     kKCoeff = 0, kKFwdH, kKFwdE, kKSample, kKQuant, kKSaveFrame, kKAdjRx, kKAdjSrc, kKMatGrad, kKAdjPmlE,
     kKAdjE, kKAdjPmlH, kKAdjH, kKTmStepFwd, kKTmStepAdj, kKTmGradReduce, kKTmSrcReduce, kKAdjWeightsE,
-    kKAdjWeightsH, kKAdjEW, kKXmFwdH, kKXmFwdE, kKXmAdjE, kKXmAdjH, kKXmPsiH, kKCount
+    kKAdjWeightsH, kKAdjEW, kKXmFwdH, kKXmFwdE, kKXmAdjE, kKXmAdjH, kKXmPsiH, kKTmStripFwd, kKTmStripAdj,
+    kKCount
 };
 
 }  // namespace dgx

@@ -1,0 +1,73 @@
+"""The 2D Ez-TM strip kernels (deepgpr_amd/csrc/dgx_tm2d_strip.hip: several
+steps a launch) against the CPU oracle, bit for bit: both shapes (few
+workgroups and many), grids smaller than a tile and with owned ranges that end
+inside, at and just past a tile edge, step counts with and without a remainder,
+unequal spacing and CPML widths, faces without CPML, PEC cells, every history
+that the 2D path keeps, and sources and coincident receivers in margins, on
+tile corners, in the CPML and on the grid's edges."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TM2D = 1 << 6
+INACTIVE_PHI = (0, 3, 4, 7, 8, 11, 12, 15)
+CASES = [
+    # (NX, NY, order, nt, nshot, S, storage, mode, pml, d, pec)
+    (14, 9, 2, 17, 1, 1, "e_only", 2, (1, 1, 1, 2), (0.02, 0.02), False),
+    (19, 23, 4, 8, 2, 1, "f32", 3, (3, 2, 4, 3), (0.02, 0.013), True),
+    (33, 49, 2, 8, 2, 3, "f32", 3, (4, 5, 0, 6), (0.017, 0.02), True),
+    (48, 96, 2, 16, 1, 2, "bf16", 3, (0, 0, 0, 0), (0.02, 0.02), False),
+    (64, 97, 2, 13, 3, 1, "f16", 2, (10, 9, 12, 11), (0.02, 0.02), True),
+    (43, 93, 4, 10, 1, 2, "bf16", 2, (0, 6, 7, 0), (0.02, 0.017), False),
+    (81, 104, 4, 7, 7, 1, "e_only", 2, (9, 10, 8, 10), (0.02, 0.02), False),
+    (101, 157, 4, 7, 9, 3, "f32", 3, (5, 3, 6, 4), (0.02, 0.016), True),
+    (61, 209, 2, 14, 14, 1, "e_only", 2, (10, 10, 10, 10), (0.02, 0.02), False),
+    (100, 105, 2, 11, 17, 2, "bf16", 3, (6, 0, 5, 7), (0.018, 0.02), True),
+]
+
+
+def _storage(h, name):
+    return {"f32": 0, "e_only": h.RHS_FROM_E, "f16": h.KIND_F16, "bf16": h.KIND_BF16}[name]
+
+
+def _problem(h, case):
+    NX, NY, order, nt, nshot, S, st, mode, pml, d, pec = case
+    p = h.make_problem(NX, NY, 2, order=order, nt=nt, nshot=nshot, nsrc=4, nrx=7, seed=31, pml=pml + (0, 0),
+                       d=d + (0.02,), pec=pec)
+    # the 2D TM contract: Ex, Ey, Hz and their CPML auxiliaries start at zero
+    for arrs, idx in ((p.E0, (0, 1)), (p.H0, (2,)), (p.lam0, (0, 1, 5))):
+        for k in idx:
+            arrs[k] = np.zeros_like(arrs[k])
+    for k in INACTIVE_PHI:
+        p.phi0[k] = np.zeros_like(p.phi0[k])
+        p.lam0[6 + k] = np.zeros_like(p.lam0[6 + k])
+    p.mode, p.S = mode, S
+    p.storage_type = _storage(h, st)
+    for s in range(nshot):
+        p.src_loc[s, 0] = [NX // 2, NY // 2, 0]
+        p.src_loc[s, 1] = [min(16 + s % 3, NX - 2), min(47 + s % 2, NY - 2), 0]
+        p.src_loc[s, 2] = p.src_loc[s, 0]
+        p.src_loc[s, 3] = [1, NY - 2, 0]
+        spots = [[NX // 2, NY // 2], [NX // 2, NY // 2], [0, 0], [NX - 2, 1], [min(20, NX - 2), min(52, NY - 2)],
+                 [min(19, NX - 2), min(51, NY - 2)], [NX // 3, NY - 2]]
+        for r, (i, j) in enumerate(spots):
+            p.rx_loc[s, r] = [i, j, 0]
+    return p
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}x{c[1]}-o{c[2]}-n{c[4]}-{c[6]}")
+def test_strips_match_oracle_bitwise(oracle_built, cuda_device, monkeypatch, case):
+    h = oracle_built
+    monkeypatch.delenv("DEEPGPR_AMD_TM2D_TILE_ROWS", raising=False)
+    print(f"[gpu strips] {case}", flush=True)
+    p = _problem(h, case)
+    cpu = h.run_cpu(p, "oracle")
+    p.storage_type |= TM2D
+    gpu = h.run_gpu(p, api="dgx")
+    bad = h.bitwise_diff(gpu, cpu, h.KEYS_FWD + ("g_src", "g_eps", "g_sig"))
+    assert not bad, bad
+    for k in [2, 3, 4] + [6 + k for k in range(24) if k not in INACTIVE_PHI]:
+        assert np.array_equal(gpu["L"][k], cpu["L"][k]), k
+    assert np.array_equal(gpu["E_saved"], cpu["E_saved"])
+    assert np.array_equal(gpu["R_saved"], cpu["R_saved"])
