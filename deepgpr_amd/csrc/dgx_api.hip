@@ -595,6 +595,20 @@ struct TuneKey {
 };
 std::mutex g_tune_mu;
 std::vector<std::pair<TuneKey, int>> g_tuned;
+// shapes that have run several steps a launch only, which has no tile rows:
+// what the one-step kernels would take untuned (dgx_tm2d_tile_rows_tuned)
+std::vector<std::pair<TuneKey, int>> g_untuned;
+
+void note_untuned(const Plan& pl)
+{
+    const char* t = std::getenv("DEEPGPR_AMD_TM2D_TUNE");
+    if (t && std::strcmp(t, "0") == 0) return;
+    const TuneKey key{pl.g.N[0], pl.g.N[1], pl.g.nshot, pl.order, pl.has_cpml ? 1 : 0};
+    std::lock_guard<std::mutex> lock(g_tune_mu);
+    for (const auto& kv : g_untuned)
+        if (kv.first == key) return;
+    g_untuned.push_back({key, tm2d_tile_rows_rule(pl)});
+}
 
 int tm2d_probe(const Plan& pl, const dgx_solve* P, hipStream_t stream, double* us_out)
 {
@@ -967,6 +981,25 @@ void strip_points(const StripMap& m, int nshot, const std::vector<int>& loc, int
     strip_lists(tmp, (long long)m.tiles * nshot, off, ent);
 }
 
+// Receiver groups (as tm_receiver_groups takes them) listed for every (tile,
+// shot) that stages the cell: (staged index, first member, member count, 0).
+void strip_groups(const StripMap& m, int nshot, int ny, const std::vector<int>& goff, const std::vector<int>& gshot,
+                  const std::vector<long long>& gcell, std::vector<int>& off, std::vector<int4>& grp)
+{
+    std::vector<std::pair<long long, int4>> tmp;
+    for (size_t q = 0; q < gshot.size(); ++q) {
+        const int i = (int)(gcell[q] / ny), j = (int)(gcell[q] % ny);
+        int a0, a1, b0, b1;
+        strip_tiles(i, m.orow, m.sh.halo, m.sh.rows, m.nti, a0, a1);
+        strip_tiles(j, m.ocol, m.sh.halo, 64, m.ntj, b0, b1);
+        for (int a = a0; a <= a1; ++a)
+            for (int b = b0; b <= b1; ++b)
+                tmp.push_back({a * m.ntj + b + (long long)m.tiles * gshot[q],
+                               make_int4(strip_local(m, a, b, i, j), goff[q], goff[q + 1] - goff[q], 0)});
+    }
+    strip_lists(tmp, (long long)m.tiles * nshot, off, grp);
+}
+
 // Receiver groups of one call: one per (shot, cell), members in receiver
 // order; cell = linear index with strides (st0, st1, 1).
 void receiver_groups(const std::vector<int>& rloc, int nshot, int nrx, long long st0, long long st1,
@@ -1118,6 +1151,7 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
     const bool strips = fused && tm2d_strips() && strip_applies(pl.order, tg0) &&
                         (P->nreceiver <= 0 || P->receiver_component == 2);
     const StripMap stm = strips ? strip_map(pl.order, tg0) : StripMap{};
+    if (strips) note_untuned(pl);
     const Tm2dGrid tg = !fused || strips ? tg0 : tm_grid_of(pl, tm2d_tile_rows(pl, P, stream));
     const int tm_tiles = (g.N[0] * g.N[1] + 255) / 256;
     long long nblocks = tm ? (long long)tm_tiles * g.nshot
@@ -1559,7 +1593,11 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
 
     const bool tm = tm2d_applies(P, pl, hsloc, hrloc);
     const bool fused = tm && tm2d_fused();
-    const Tm2dGrid tg = tm_grid_of(pl, fused ? tm2d_tile_rows(pl, P, stream) : kTmBI);
+    const Tm2dGrid tg0 = tm_grid_of(pl, kTmBI);
+    const bool strips = fused && tm2d_strips() && strip_applies(pl.order, tg0);
+    const StripMap stm = strips ? strip_map(pl.order, tg0) : StripMap{};
+    if (strips) note_untuned(pl);
+    const Tm2dGrid tg = !fused || strips ? tg0 : tm_grid_of(pl, tm2d_tile_rows(pl, P, stream));
     Grid gc = g;  // compact 2D TM addressing for the receiver/source kernels
     if (tm) {
         gc.st0 = g.N[1];
@@ -1626,7 +1664,8 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
     if (fused && adj_rx && !gshot.empty()) {
         std::vector<int> xoff;
         std::vector<int4> xgrp;
-        tm_receiver_groups(tg, pl.order, goff, gshot, gcell, xoff, xgrp);
+        if (strips) strip_groups(stm, g.nshot, tg.NY, goff, gshot, gcell, xoff, xgrp);
+        else tm_receiver_groups(tg, pl.order, goff, gshot, gcell, xoff, xgrp);
         if (!upload(d_xoff, xoff, stream) || !upload(d_xgrp, xgrp, stream)) {
             set_error("backward: out of device memory for receiver lists");
             return -1;
@@ -1646,7 +1685,8 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
     if (fused && want_src) {
         std::vector<int> soff;
         std::vector<int2> sent;
-        tm_source_lists(tg, hsloc, P->nsource, soff, sent);
+        if (strips) strip_points(stm, g.nshot, hsloc, P->nsource, false, soff, sent);
+        else tm_source_lists(tg, hsloc, P->nsource, soff, sent);
         if (!upload(d_soff, soff, stream) || !upload(d_sent, sent, stream) ||
             !d_svals.alloc((size_t)nt * g.nshot * P->nsource * sizeof(float))) {
             set_error("backward: out of device memory for source lists");
@@ -1658,9 +1698,16 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
         tgrad.src_vals = (float*)d_svals.p;
         tgrad.nsrc = P->nsource;
     }
-    // two buffers: a launch writes one while it sums the other (the previous saved step)
+    // Two buffers: a launch writes one while it sums the other (the previous
+    // saved step). The strip kernels write up to strip_saves saved steps of
+    // several shots and the sum kernel adds them; their buffers take no more
+    // than two did, or 32 MiB.
     const long long terms_len = 2 * (long long)g.nshot * pl.box.cells;
-    if (fused && want_mat && !d_terms.alloc((size_t)2 * terms_len * sizeof(float))) {
+    const int strip_saves =
+        strips ? (int)std::min<long long>(stm.sh.steps, std::max<long long>(2, (8LL << 20) / std::max(terms_len, 1LL)))
+               : 2;
+    if (fused && want_mat && !(strips && g.nshot == 1) &&
+        !d_terms.alloc((size_t)strip_saves * terms_len * sizeof(float))) {
         set_error("backward: out of device memory for per-shot gradient terms");
         return -1;
     }
@@ -1815,7 +1862,48 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
     tgrad.gsig = gsig;
     tgrad.mg = mg;
     int terms_buf = 0;
-    for (int it = nt - 1; it >= 0; --it) {
+    if (strips) {
+        StripGrad sg{};
+        sg.on = want_mat;
+        sg.kind = pl.kind;
+        sg.e_only = pl.e_only;
+        sg.S = std::max(S, 1);
+        sg.nt = nt;
+        sg.nt_saved = pl.nt_saved;
+        sg.e = P->E_saved;
+        sg.r = P->R_saved;
+        sg.snap = pl.snap;
+        sg.eoff = tgrad.ez_comp * pl.cstride;
+        sg.roff = tgrad.ez_comp * pl.snap;
+        sg.sig = P->sigma_pad;
+        sg.dt = P->dt;
+        sg.want_eps = mg.want_eps;
+        sg.want_sig = mg.want_sig;
+        sg.box = pl.box;
+        sg.terms = (float*)d_terms.p;
+        sg.terms_len = terms_len;
+        sg.geps = geps;
+        sg.gsig = gsig;
+        sg.src_vals = tgrad.src_vals;
+        sg.nsrc = tgrad.nsrc;
+        sg.geo = geo;
+        for (int it = nt - 1; it >= 0;) {
+            int nsub = std::min(stm.sh.steps, it + 1);
+            // saved steps among it - nsub + 1 .. it: multiples of S
+            auto saves = [&](int n) { return want_mat ? it / sg.S - (it - n + sg.S) / sg.S + 1 : 0; };
+            if (g.nshot > 1)
+                while (saves(nsub) > strip_saves) --nsub;
+            TIMED(tmr, kKTmStripAdj,
+                  launch_tm_strip_adj(pl.order, tms.g, tms.f, tms.pp, stm, tsrc, tax, sg, it, nsub, fp64, stream));
+            tms.flip();
+            if (g.nshot > 1 && saves(nsub) > 0)
+                TIMED(tmr, kKTmGradReduce,
+                      launch_tm_grad_reduce(tms.g, pl.box, sg.terms, saves(nsub), terms_len, mg.want_eps, mg.want_sig,
+                                            geps, gsig, fp64, stream));
+            it -= nsub;
+        }
+    }
+    for (int it = strips ? -1 : nt - 1; it >= 0; --it) {
         if (fused) {
             tgrad.pending = tgrad.terms;
             tgrad.terms = nullptr;
@@ -1893,7 +1981,8 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
     }
     if (fused && tgrad.terms)  // the last saved step has no later launch to sum it
         TIMED(tmr, kKTmGradReduce,
-              launch_tm_grad_reduce(tms.g, pl.box, tgrad.terms, mg.want_eps, mg.want_sig, geps, gsig, fp64, stream));
+              launch_tm_grad_reduce(tms.g, pl.box, tgrad.terms, 1, terms_len, mg.want_eps, mg.want_sig, geps, gsig,
+                                    fp64, stream));
     if (fused && want_src)
         TIMED(tmr, kKTmSrcReduce,
               launch_tm_src_reduce(tgrad.src_vals, P->grad_source, g.nshot, P->nsource, nt, stream));
@@ -2367,7 +2456,7 @@ int batch_phase_end(Batch* b, BatchInstance& I, bool& finished)
     if (d.phase == 1) {
         // the last saved step (it = 0) has no later launch to sum it
         const float* last = d.terms + (size_t)((d.nt - 1) & 1) * d.terms_len;
-        launch_tm_grad_reduce(d.g, d.box, last, d.want_eps, d.want_sig, d.geps, d.gsig, true, stream);
+        launch_tm_grad_reduce(d.g, d.box, last, 1, d.terms_len, d.want_eps, d.want_sig, d.geps, d.gsig, true, stream);
         if (d.want_eps) launch_add_f64(d.geps, I.grad_eps, I.ngrad, stream);
         if (d.want_sig) launch_add_f64(d.gsig, I.grad_sig, I.ngrad, stream);
     }
@@ -2450,8 +2539,9 @@ DGX_API int dgx_tm2d_tile_rows_tuned(int nx_fields, int ny_fields, int nshot, in
 {
     const TuneKey key{nx_fields, ny_fields, nshot, order, cpml ? 1 : 0};
     std::lock_guard<std::mutex> lock(g_tune_mu);
-    for (const auto& kv : g_tuned)
-        if (kv.first == key) return kv.second;
+    for (const auto* list : {&g_tuned, &g_untuned})
+        for (const auto& kv : *list)
+            if (kv.first == key) return kv.second;
     return 0;
 }
 

@@ -251,8 +251,8 @@ void launch_step_counter(int* it, int value, bool add, hipStream_t st);
 void launch_tm_step_adj(int order, const Tm2dGrid& g, const Tm2dFields& f, const TmPingPong& pp,
                         const SourceBlocks& src, const TmReceiversAdj& rx, const TmAdjGrad& ag, int it, bool fp64,
                         hipStream_t st);
-void launch_tm_grad_reduce(const Tm2dGrid& g, const Box& b, const float* terms, int want_eps, int want_sig,
-                           void* geps, void* gsig, bool fp64, hipStream_t st);
+void launch_tm_grad_reduce(const Tm2dGrid& g, const Box& b, const float* terms, int steps, long long terms_len,
+                           int want_eps, int want_sig, void* geps, void* gsig, bool fp64, hipStream_t st);
 void launch_tm_src_reduce(const float* vals, float* gsrc, int nshot, int nsrc, int nt, hipStream_t st);
 
 // Strip kernels: several steps a launch (dgx_tm2d_strip.hip). Source and
@@ -265,11 +265,32 @@ struct StripHist {
     long long cstride;   // elements between components
     Box box;
 };
+// Adjoint: history, material terms and source values of a launch.
+struct StripGrad {
+    int on;                  // material gradients are wanted
+    int kind, e_only, S, nt, nt_saved;
+    const void *e, *r;       // E frames; R frames or (e_only) the last E frame
+    long long snap;          // elements of one frame of one component
+    long long eoff, roff;    // offset of the Ez component in e (and R frames), in the last E frame
+    const float* sig;
+    float dt;
+    int want_eps, want_sig;
+    Box box;
+    float* terms;            // several shots: terms_len per-shot terms a saved step
+    long long terms_len;
+    void *geps, *gsig;       // one shot: the sums
+    float* src_vals;         // per (step, shot, source)
+    int nsrc;
+    float geo;
+};
 bool strip_applies(int order, const Tm2dGrid& g);
 StripMap strip_map(int order, const Tm2dGrid& g);
 void launch_tm_strip_fwd(int order, const Tm2dGrid& g, const Tm2dFields& f, const TmPingPong& pp, const StripMap& sm,
                          const SourceBlocks& src, const TmReceiversFwd& rx, const StripHist& hist, int it0, int nsub,
                          hipStream_t st);
+void launch_tm_strip_adj(int order, const Tm2dGrid& g, const Tm2dFields& f, const TmPingPong& pp, const StripMap& sm,
+                         const SourceBlocks& src, const TmReceiversAdj& rx, const StripGrad& mg, int it0, int nsub,
+                         bool fp64, hipStream_t st);
 
 void launch_tm_fwd_h(int order, const Tm2dGrid& g, const Tm2dFields& f, hipStream_t st);
 void launch_tm_fwd_e(int order, const Tm2dGrid& g, const Tm2dFields& f, const SourceBlocks& src,

@@ -12,6 +12,7 @@
 namespace dgx {
 
 struct StripShape {
+    int size;    // which of the shapes (dgx_tm2d_strip.hip)
     int rows;    // SR
     int halo;    // H
     int steps;   // T

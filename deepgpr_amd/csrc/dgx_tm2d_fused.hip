@@ -162,19 +162,6 @@ __device__ __forceinline__ long long terms_out(const Tm2dGrid& g, const Box& b, 
     return (long long)i * (g.NY - 1) + j;
 }
 
-// Sum of the per-shot material terms of cell h of the history box, in shot
-// order, added to the accumulators (one saved step).
-template <typename ACC>
-__device__ __forceinline__ void reduce_terms(const Tm2dGrid& g, const Box& b, const float* __restrict__ terms,
-                                             long long h, int want_eps, int want_sig, ACC* __restrict__ geps,
-                                             ACC* __restrict__ gsig)
-{
-    const long long out = terms_out(g, b, h);
-    const long long sstride = (long long)g.nshot * b.cells;
-    if (want_eps) geps[out] += sum_shots<ACC>(terms + h, b.cells, g.nshot);
-    if (want_sig) gsig[out] += sum_shots<ACC>(terms + sstride + h, b.cells, g.nshot);
-}
-
 template <int ORDER, typename ACC, int TBI>
 __global__ __launch_bounds__(NTA) void k_tm_step_adj(Tm2dGrid g, Tm2dFields f, TmPingPong pp, SourceBlocks src,
                                                      TmReceiversAdj rx, TmAdjGrad ag, int it)
@@ -186,15 +173,21 @@ __global__ __launch_bounds__(NTA) void k_tm_step_adj(Tm2dGrid g, Tm2dFields f, T
 #include "dgx_tm2d_tile_adj.inc"
 }
 
-// Material gradient of one saved step: per-shot terms summed in shot order.
+// Material gradients of `steps` saved steps, terms_len terms each: per-shot
+// terms summed in shot order, the steps added in order.
 template <typename ACC>
-__global__ __launch_bounds__(256) void k_tm_grad_reduce(Tm2dGrid g, Box b, const float* __restrict__ terms,
-                                                        int want_eps, int want_sig, ACC* __restrict__ geps,
-                                                        ACC* __restrict__ gsig)
+__global__ __launch_bounds__(256) void k_tm_grad_reduce(Tm2dGrid g, Box b, const float* __restrict__ terms, int steps,
+                                                        long long terms_len, int want_eps, int want_sig,
+                                                        ACC* __restrict__ geps, ACC* __restrict__ gsig)
 {
     const long long h = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= b.cells) return;
-    reduce_terms<ACC>(g, b, terms, h, want_eps, want_sig, geps, gsig);
+    const bool sig = blockIdx.y;
+    if (h >= b.cells || !(sig ? want_sig : want_eps)) return;
+    ACC* acc = (sig ? gsig : geps) + terms_out(g, b, h);
+    const float* t = terms + (sig ? (long long)g.nshot * b.cells : 0) + h;
+    ACC sum = *acc;
+    for (int k = 0; k < steps; ++k) sum += sum_shots<ACC>(t + k * terms_len, b.cells, g.nshot);
+    *acc = sum;
 }
 
 // grad_source[k, it] += per-shot values, shots in order
@@ -484,17 +477,17 @@ void launch_tm_step_adj(int order, const Tm2dGrid& g, const Tm2dFields& f, const
     }
 }
 
-void launch_tm_grad_reduce(const Tm2dGrid& g, const Box& b, const float* terms, int want_eps, int want_sig,
-                           void* geps, void* gsig, bool fp64, hipStream_t st)
+void launch_tm_grad_reduce(const Tm2dGrid& g, const Box& b, const float* terms, int steps, long long terms_len,
+                           int want_eps, int want_sig, void* geps, void* gsig, bool fp64, hipStream_t st)
 {
     if (b.cells <= 0) return;
     const unsigned blocks = (unsigned)((b.cells + 255) / 256);
     if (fp64)
-        hipLaunchKernelGGL(k_tm_grad_reduce<double>, dim3(blocks), dim3(256), 0, st, g, b, terms, want_eps,
-                           want_sig, (double*)geps, (double*)gsig);
+        hipLaunchKernelGGL(k_tm_grad_reduce<double>, dim3(blocks, 2), dim3(256), 0, st, g, b, terms, steps,
+                           terms_len, want_eps, want_sig, (double*)geps, (double*)gsig);
     else
-        hipLaunchKernelGGL(k_tm_grad_reduce<float>, dim3(blocks), dim3(256), 0, st, g, b, terms, want_eps,
-                           want_sig, (float*)geps, (float*)gsig);
+        hipLaunchKernelGGL(k_tm_grad_reduce<float>, dim3(blocks, 2), dim3(256), 0, st, g, b, terms, steps,
+                           terms_len, want_eps, want_sig, (float*)geps, (float*)gsig);
 }
 
 void launch_tm_src_reduce(const float* vals, float* gsrc, int nshot, int nsrc, int nt, hipStream_t st)

@@ -128,7 +128,9 @@ DGX_API long long dgx_forward_noalloc_scratch_bytes(void);
  * nx_fields x ny_fields, shots, FDTD order, CPML present), or 0 when no solve
  * of that shape has run yet in this process. The first solve of a shape times
  * the forward step kernel at each height on buffers of its own and keeps the
- * fastest; every height gives the same results. */
+ * fastest; every height gives the same results. A shape whose solves advance
+ * several steps a launch (orders 2 and 4) has no use for it and is not timed:
+ * it reports the height that the rule by size gives. */
 DGX_API int dgx_tm2d_tile_rows_tuned(int nx_fields, int ny_fields, int nshot, int order, int cpml);
 /* FP16/BF16 history codec round trip on device arrays; replaces
  * deepgpr_test_wavefield_conversion (deepgpr.h:84-86). */

@@ -1,10 +1,10 @@
 """The 2D Ez-TM strip kernels (deepgpr_amd/csrc/dgx_tm2d_strip.hip: several
-steps a launch) against the CPU oracle, bit for bit: both shapes (few
-workgroups and many), grids smaller than a tile and with owned ranges that end
-inside, at and just past a tile edge, step counts with and without a remainder,
-unequal spacing and CPML widths, faces without CPML, PEC cells, every history
-that the 2D path keeps, and sources and coincident receivers in margins, on
-tile corners, in the CPML and on the grid's edges."""
+steps a launch) against the CPU oracle, bit for bit: every shape (few
+workgroups and many, one shot and several), grids smaller than a tile and with
+owned ranges that end inside, at and just past a tile edge, step counts with
+and without a remainder, unequal spacing and CPML widths, faces without CPML,
+PEC cells, every history that the 2D path keeps, and sources and coincident
+receivers in margins, on tile corners, in the CPML and on the grid's edges."""
 import numpy as np
 import pytest
 
@@ -24,6 +24,10 @@ CASES = [
     (101, 157, 4, 7, 9, 3, "f32", 3, (5, 3, 6, 4), (0.02, 0.016), True),
     (61, 209, 2, 14, 14, 1, "e_only", 2, (10, 10, 10, 10), (0.02, 0.02), False),
     (100, 105, 2, 11, 17, 2, "bf16", 3, (6, 0, 5, 7), (0.018, 0.02), True),
+    (61, 209, 4, 5, 26, 1, "bf16", 2, (6, 9, 10, 5), (0.02, 0.02), False),
+    (64, 105, 2, 8, 43, 2, "f32", 3, (6, 9, 10, 5), (0.02, 0.019), True),
+    (300, 700, 2, 9, 1, 2, "f32", 3, (10, 7, 9, 10), (0.02, 0.02), True),
+    (251, 731, 4, 5, 1, 1, "e_only", 2, (10, 7, 9, 10), (0.02, 0.021), False),
 ]
 
 
