@@ -2051,6 +2051,8 @@ struct BatchInstance {
     int order = 2;
     bool gradient = false;
     TmBatchInst d{};
+    bool strip = false;   // several steps a launch (dgx_tm2d_strip.hip)
+    StripBatchInst sd{};  // then its arguments
     Tm2dState tms;
     DevBuf l_soff, l_sent, l_roff, l_rent, l_xoff, l_xgrp, l_mem;
     DevBuf dgrad, acc, terms;
@@ -2106,13 +2108,18 @@ struct Batch {
     std::vector<std::pair<int, hipEvent_t>> finished;
     RetireList<HipRetireOps, Retiree> retired;
     bool dirty = true;
-    std::unique_ptr<DevBuf> table;  // descriptors and prefixes of the 6 slots
+    std::unique_ptr<DevBuf> table;  // descriptors and prefixes of the slots
     size_t table_cap = 0;
     Staging ring[8];
     int ring_next = 0;
     const TmBatchInst* desc[6] = {};
     const int* prefix[6] = {};
     int ninst[6] = {}, total[6] = {}, order_of[6] = {2, 4, 8, 2, 4, 8};
+    // the strip instances: slots of orders 2 and 4, forward then adjoint, and the
+    // launches of each order so far
+    StripBatchSlot strip[4] = {};
+    int slaunch[2] = {};
+    bool strips() const { return strip[0].ninst || strip[1].ninst || strip[2].ninst || strip[3].ninst; }
     // kBatchGraphSteps steps of the current table as one graph (kernel nodes
     // only); node q launches step *gbase + q
     DevBuf gbase;
@@ -2195,6 +2202,7 @@ bool batch_graph_ready(Batch* b)
 }
 
 int order_slot(int order) { return order == 8 ? 2 : (order == 4 ? 1 : 0); }
+int strip_slot(const BatchInstance& I) { return order_slot(I.order) + 2 * I.d.phase; }
 
 // Moves memory the batch stream may still read to the retired list, behind
 // an event recorded on the batch stream now (after every launch queued so
@@ -2267,8 +2275,16 @@ int batch_add(Batch* b, const dgx_solve* P, const dgx_solve* G, hipStream_t stre
     d.pp = I.tms.pp;
     std::vector<int> soff, roff;
     std::vector<int2> sent, rent;
-    tm_source_lists(tg, hsloc, P->nsource, soff, sent);
-    tm_receiver_lists(tg, hrloc, P->nreceiver, roff, rent);
+    // one shot: its sums need no terms of other shots, so its launches may hold several steps
+    I.strip = g.nshot == 1 && tm2d_strips() && strip_applies(pl.order, tg);
+    const StripMap stm = I.strip ? strip_batch_map(pl.order, tg) : StripMap{};
+    if (I.strip) {
+        strip_points(stm, 1, hsloc, P->nsource, true, soff, sent);
+        strip_points(stm, 1, hrloc, P->nreceiver, false, roff, rent);
+    } else {
+        tm_source_lists(tg, hsloc, P->nsource, soff, sent);
+        tm_receiver_lists(tg, hrloc, P->nreceiver, roff, rent);
+    }
     if (!upload(I.l_soff, soff, stream) || !upload(I.l_sent, sent, stream) || !upload(I.l_roff, roff, stream) ||
         !upload(I.l_rent, rent, stream)) {
         set_error("batch: out of device memory for lists");
@@ -2314,7 +2330,8 @@ int batch_add(Batch* b, const dgx_solve* P, const dgx_solve* G, hipStream_t stre
         std::vector<long long> gcell;
         std::vector<int4> xgrp;
         receiver_groups(hrloc, g.nshot, P->nreceiver, g.N[1], 1, goff, gshot, gcell, gmem);
-        tm_receiver_groups(tg, pl.order, goff, gshot, gcell, xoff, xgrp);
+        if (I.strip) strip_groups(stm, 1, tg.NY, goff, gshot, gcell, xoff, xgrp);
+        else tm_receiver_groups(tg, pl.order, goff, gshot, gcell, xoff, xgrp);
         if (!upload(I.l_xoff, xoff, stream) || !upload(I.l_xgrp, xgrp, stream) || !upload(I.l_mem, gmem, stream) ||
             !I.dgrad.alloc((size_t)I.rx_count * sizeof(float))) {
             set_error("batch: out of device memory for receiver groups");
@@ -2330,7 +2347,7 @@ int batch_add(Batch* b, const dgx_solve* P, const dgx_solve* G, hipStream_t stre
         I.ngrad = (long long)(g.N[0] - 1) * (g.N[1] - 1) * (g.N[2] - 1);
         d.terms_len = 2 * (long long)g.nshot * pl.box.cells;
         if (!I.acc.alloc((size_t)I.ngrad * 2 * sizeof(double)) ||
-            !I.terms.alloc((size_t)2 * d.terms_len * sizeof(float))) {
+            (!I.strip && !I.terms.alloc((size_t)2 * d.terms_len * sizeof(float)))) {
             set_error("batch: out of device memory for gradient accumulators");
             return -1;
         }
@@ -2341,6 +2358,56 @@ int batch_add(Batch* b, const dgx_solve* P, const dgx_solve* G, hipStream_t stre
     }
     d.phase = 0;
     d.start = b->gstep;
+    if (I.strip) {
+        const Spacing sx = make_spacing(g.d[0]), sy = make_spacing(g.d[1]);
+        StripArgs& fa = I.sd.fwd;
+        fa.g = tg;
+        fa.f = d.f;
+        fa.pp = d.pp;
+        fa.sm = stm;
+        fa.src = d.src;
+        fa.rx = d.rx;
+        fa.hist.on = gradient;
+        fa.hist.kind = d.kind;
+        fa.hist.mode = d.mode;
+        fa.hist.S = 1;
+        fa.hist.e = d.e_saved;
+        fa.hist.snap = d.snap;
+        fa.hist.cstride = d.cstride;
+        fa.hist.box = d.box;
+        fa.sx = sx;
+        fa.sy = sy;
+        StripAdjArgs& aa = I.sd.adj;
+        aa.g = tg;
+        aa.f = d.f;
+        aa.pp = d.pp;
+        aa.sm = stm;
+        aa.rx = d.rxa;
+        aa.inv[0] = 1.0f / g.d[0];
+        aa.inv[1] = 1.0f / g.d[1];
+        StripGrad& mg = aa.mg;
+        mg.on = gradient && (d.want_eps || d.want_sig);
+        mg.kind = d.kind;
+        mg.e_only = 1;
+        mg.S = 1;
+        mg.nt = d.nt;
+        mg.nt_saved = d.nt_saved;
+        mg.e = d.e_saved;
+        mg.r = d.e_final;
+        mg.snap = d.snap;
+        mg.eoff = d.mode == 3 ? 2 * d.cstride : 0;
+        mg.roff = d.mode == 3 ? 2 * d.snap : 0;
+        mg.sig = d.sig_full;
+        mg.dt = d.dt;
+        mg.want_eps = d.want_eps;
+        mg.want_sig = d.want_sig;
+        mg.box = d.box;
+        mg.geps = d.geps;
+        mg.gsig = d.gsig;
+        I.sd.nt = d.nt;
+        I.sd.start = b->gstep;
+        I.sd.launch = b->slaunch[order_slot(I.order)];
+    }
     DGX_TRY(hipGetLastError(), "batch: kernel launch");
     if (stream != b->stream) {
         hipEvent_t ready;
@@ -2367,7 +2434,7 @@ int batch_rebuild(Batch* b)
         prefix[slot].assign(1, 0);
         for (auto& ip : b->active) {
             const BatchInstance& I = *ip;
-            if (order_slot(I.order) + 3 * I.d.phase != slot) continue;
+            if (I.strip || order_slot(I.order) + 3 * I.d.phase != slot) continue;
             desc[slot].push_back(I.d);
             prefix[slot].push_back(prefix[slot].back() + I.d.g.ftiles * I.d.g.nshot);
         }
@@ -2377,6 +2444,24 @@ int batch_rebuild(Batch* b)
         bytes = align(bytes + desc[slot].size() * sizeof(TmBatchInst));
         off_prefix[slot] = bytes;
         bytes = align(bytes + prefix[slot].size() * sizeof(int));
+    }
+    std::vector<StripBatchInst> sdesc[4];
+    std::vector<int> sprefix[4];
+    size_t off_sdesc[4], off_sprefix[4];
+    for (int slot = 0; slot < 4; ++slot) {
+        sprefix[slot].assign(1, 0);
+        for (auto& ip : b->active) {
+            const BatchInstance& I = *ip;
+            if (!I.strip || strip_slot(I) != slot) continue;
+            sdesc[slot].push_back(I.sd);
+            sprefix[slot].push_back(sprefix[slot].back() + I.sd.fwd.sm.tiles);
+        }
+        b->strip[slot].ninst = (int)sdesc[slot].size();
+        b->strip[slot].total = sprefix[slot].back();
+        off_sdesc[slot] = bytes;
+        bytes = align(bytes + sdesc[slot].size() * sizeof(StripBatchInst));
+        off_sprefix[slot] = bytes;
+        bytes = align(bytes + sprefix[slot].size() * sizeof(int));
     }
     if (bytes > b->table_cap) {
         // queued steps still read the old table: retire it behind an event
@@ -2408,6 +2493,12 @@ int batch_rebuild(Batch* b)
         b->desc[slot] = (const TmBatchInst*)(dv + off_desc[slot]);
         b->prefix[slot] = (const int*)(dv + off_prefix[slot]);
     }
+    for (int slot = 0; slot < 4; ++slot) {
+        std::memcpy(h + off_sdesc[slot], sdesc[slot].data(), sdesc[slot].size() * sizeof(StripBatchInst));
+        std::memcpy(h + off_sprefix[slot], sprefix[slot].data(), sprefix[slot].size() * sizeof(int));
+        b->strip[slot].insts = (const StripBatchInst*)(dv + off_sdesc[slot]);
+        b->strip[slot].prefix = (const int*)(dv + off_sprefix[slot]);
+    }
     if (hipMemcpyAsync(dv, h, bytes, hipMemcpyHostToDevice, b->stream) != hipSuccess ||
         hipEventRecord(r.done, b->stream) != hipSuccess)
         return -1;
@@ -2424,7 +2515,8 @@ int batch_phase_end(Batch* b, BatchInstance& I, bool& finished)
     finished = false;
     if (d.phase == 0 && I.gradient) {
         const long long field = (long long)d.g.nshot * d.g.plane;
-        const float* ez = (d.nt & 1) ? d.pp.Ez[1] : d.pp.Ez[0];
+        const int copy = I.strip ? (b->slaunch[order_slot(I.order)] - I.sd.launch) & 1 : d.nt & 1;
+        const float* ez = d.pp.Ez[copy];
         HistWrite hw{};
         hw.mode = d.mode;
         hw.box = d.box;
@@ -2451,12 +2543,17 @@ int batch_phase_end(Batch* b, BatchInstance& I, bool& finished)
         launch_clear_spans(sp, stream);
         d.phase = 1;
         d.start = b->gstep;
+        I.sd.start = b->gstep;
+        if (I.strip) I.sd.launch = b->slaunch[order_slot(I.order)];
         return 0;
     }
     if (d.phase == 1) {
         // the last saved step (it = 0) has no later launch to sum it
-        const float* last = d.terms + (size_t)((d.nt - 1) & 1) * d.terms_len;
-        launch_tm_grad_reduce(d.g, d.box, last, 1, d.terms_len, d.want_eps, d.want_sig, d.geps, d.gsig, true, stream);
+        if (!I.strip) {
+            const float* last = d.terms + (size_t)((d.nt - 1) & 1) * d.terms_len;
+            launch_tm_grad_reduce(d.g, d.box, last, 1, d.terms_len, d.want_eps, d.want_sig, d.geps, d.gsig, true,
+                                  stream);
+        }
         if (d.want_eps) launch_add_f64(d.geps, I.grad_eps, I.ngrad, stream);
         if (d.want_sig) launch_add_f64(d.gsig, I.grad_sig, I.ngrad, stream);
     }
@@ -2481,7 +2578,22 @@ int batch_step(Batch* b, int steps)
         long long room = std::numeric_limits<long long>::max();
         for (const auto& ip : b->active) room = std::min<long long>(room, (long long)ip->d.start + ip->d.nt - b->gstep);
         int adv = 1;
-        if (batch_graphs() && room >= kBatchGraphSteps && steps - k >= kBatchGraphSteps && batch_graph_ready(b)) {
+        if (b->strips()) {
+            // as many steps as the longest launch holds; shorter launches and
+            // one-step launches repeat
+            adv = (int)std::min<long long>({room, steps - k, std::max(strip_batch_steps(2), strip_batch_steps(4))});
+            for (int slot = 0; slot < 2; ++slot) {
+                const int order = slot ? 4 : 2, most = strip_batch_steps(order);
+                if (b->strip[slot].total + b->strip[slot + 2].total == 0) continue;
+                for (int q = 0; q < adv; q += most)
+                    launch_tm_strip_batch(order, b->strip[slot], b->strip[slot + 2], b->gstep + q, b->slaunch[slot]++,
+                                          std::min(most, adv - q), b->stream);
+            }
+            for (int q = 0; q < adv; ++q)
+                for (int slot = 0; slot < 6; ++slot)
+                    launch_tm_batch(b->order_of[slot], slot >= 3, b->desc[slot], b->prefix[slot], b->ninst[slot],
+                                    b->total[slot], b->gstep + q, b->stream);
+        } else if (batch_graphs() && room >= kBatchGraphSteps && steps - k >= kBatchGraphSteps && batch_graph_ready(b)) {
             launch_step_counter((int*)b->gbase.p, b->gstep, false, b->stream);
             DGX_TRY(hipGraphLaunch(b->gexec, b->stream), "batch: graph launch");
             adv = kBatchGraphSteps;

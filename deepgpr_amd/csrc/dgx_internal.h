@@ -283,7 +283,48 @@ struct StripGrad {
     int nsrc;
     float geo;
 };
+struct StripArgs {
+    Tm2dGrid g;
+    Tm2dFields f;
+    TmPingPong pp;
+    StripMap sm;
+    SourceBlocks src;
+    TmReceiversFwd rx;
+    StripHist hist;
+    Spacing sx, sy;
+    int it0, nsub, frame;  // steps it0 .. it0 + nsub - 1, the first history frame not yet written
+};
+struct StripAdjArgs {
+    Tm2dGrid g;
+    Tm2dFields f;
+    TmPingPong pp;
+    StripMap sm;
+    SourceBlocks src;
+    TmReceiversAdj rx;
+    StripGrad mg;
+    float inv[2];
+    int it0, nsub, frame;  // steps it0 .. it0 - nsub + 1, the newest saved step's frame
+};
+// A one-shot instance of a batch (history at every step, FP64 sums): steps and
+// state copies follow from the batch's step and launch counters.
+struct StripBatchInst {
+    StripArgs fwd;
+    StripAdjArgs adj;
+    int nt;
+    int start, launch;  // step and launch count (of its order) at which the phase started
+};
+// The instances of one order and phase: prefix[k] .. prefix[k + 1] are the
+// workgroups of instance k.
+struct StripBatchSlot {
+    const StripBatchInst* insts;
+    const int* prefix;
+    int ninst, total;
+};
 bool strip_applies(int order, const Tm2dGrid& g);
+StripMap strip_batch_map(int order, const Tm2dGrid& g);
+int strip_batch_steps(int order);  // steps a launch, at most
+void launch_tm_strip_batch(int order, const StripBatchSlot& fwd, const StripBatchSlot& adj, int gstep, int launch,
+                           int nsub, hipStream_t st);
 StripMap strip_map(int order, const Tm2dGrid& g);
 void launch_tm_strip_fwd(int order, const Tm2dGrid& g, const Tm2dFields& f, const TmPingPong& pp, const StripMap& sm,
                          const SourceBlocks& src, const TmReceiversFwd& rx, const StripHist& hist, int it0, int nsub,

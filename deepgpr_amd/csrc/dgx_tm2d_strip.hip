@@ -61,7 +61,8 @@ __device__ __forceinline__ T choose(bool c, T a, T b)
     return c ? a : b;
 }
 
-__device__ __forceinline__ StripFace strip_face(const Tm2dGrid& g, bool electric, int axis, bool high)
+template <typename G>
+__device__ __forceinline__ StripFace strip_face(const G& g, bool electric, int axis, bool high)
 {
     StripFace o;
     const int n = axis == 0 ? g.NX : g.NY;
@@ -77,7 +78,8 @@ __device__ __forceinline__ Cpml4 cpml_profile(const float* R, int p, int q)
     return {R[q] - 1.0f, R[p + q], R[2 * p + q], R[3 * p + q]};
 }
 
-__device__ __forceinline__ float axis_k(const Tm2dGrid& g, float c1, int a)
+template <typename G>
+__device__ __forceinline__ float axis_k(const G& g, float c1, int a)
 {
     if (a == 0 || g.d[a] == g.d[0]) return c1;
     return c1 * g.d[0] / g.d[a];
@@ -205,41 +207,31 @@ __device__ __forceinline__ void exchange(const float (&v)[KR], float (*first)[DN
 // One barrier per half step (its first and last rows through LDS) and one more
 // where the tile owns a receiver. A source is added by every tile that stages
 // its cell, a receiver read by the tile that owns it.
-struct StripArgs {
-    Tm2dGrid g;
-    Tm2dFields f;
-    TmPingPong pp;
-    StripMap sm;
-    SourceBlocks src;
-    TmReceiversFwd rx;
-    StripHist hist;
-    Spacing sx, sy;
-    int it0, nsub, frame;  // steps it0 .. it0 + nsub - 1, the first history frame not yet written
-};
-
-// The kernel's arguments, read where they are used: what only the stores or a
-// listed source need is not kept in scalar registers over the steps.
+// The arguments are read where they are used: what only the stores or a listed
+// source need is not kept in scalar registers over the steps.
 typedef const __attribute__((address_space(4))) StripArgs* StripArgsPtr;
-__device__ __forceinline__ StripArgsPtr args_now()
+typedef const __attribute__((address_space(4))) StripAdjArgs* StripAdjArgsPtr;
+template <typename P>
+__device__ __forceinline__ P again(P a)
 {
-    StripArgsPtr a = (StripArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(a));
     return a;
 }
 
+// Tile (ti, tj) of shot s, steps it0 .. it0 + nsub - 1; frame: the first history
+// frame not yet written; par: which copy of the state holds step it0.
 template <int ORDER, int KR, int NW, int T>
-__global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
+__device__ __forceinline__ void strip_fwd(StripArgsPtr args, int ti, int tj, int s, int it0, int nsub, int frame,
+                                          int par)
 {
-    const Tm2dGrid& g = args.g;
-    const Tm2dFields& f = args.f;
-    const TmPingPong& pp = args.pp;
-    const StripMap& sm = args.sm;
-    const StripHist& hist = args.hist;
-    const Spacing &sx = args.sx, &sy = args.sy;
-    const int it0 = args.it0, nsub = args.nsub;
+    const auto& g = args->g;
+    const auto& f = args->f;
+    const auto& pp = args->pp;
+    const auto& sm = args->sm;
+    const auto& hist = args->hist;
+    const Spacing sx{args->sx.d, args->sx.y, args->sx.big}, sy{args->sy.d, args->sy.y, args->sy.big};
     using St = Strip<ORDER, KR, NW, T>;
     constexpr int R = St::R, H = St::H, SR = St::SR;
-    const int tj = blockIdx.x, ti = blockIdx.y, s = blockIdx.z;
     const int tile = ti * sm.ntj + tj;
     __shared__ float e_first[NW][R][64], e_last[NW][R > 1 ? R - 1 : 1][64];
     __shared__ float h_first[NW][R > 1 ? R - 1 : 1][64], h_last[NW][R][64];
@@ -258,7 +250,7 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
 
     float ez[KR], hx[KR], hy[KR], ca[KR], cc[KR], cb[KR], hc[KR], hr[KR];
     float pxe[KR], pye[KR], pxh[KR], pyh[KR];
-    const float *gez = pp.Ez[0] + sb, *ghx = pp.Hx[0] + sb, *ghy = pp.Hy[0] + sb;
+    const float *gez = pp.Ez[par] + sb, *ghx = pp.Hx[par] + sb, *ghy = pp.Hy[par] + sb;
 #pragma unroll
     for (int q = 0; q < KR; ++q) {
         const unsigned p = 4u * (unsigned)(min(max(i0 + q, 0), g.NX - 1) * g.NY + cj);
@@ -287,24 +279,24 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
         for (int q = 0; q < KR; ++q) hr[q] = ld(f.hrhs, 4u * (unsigned)(min(max(i0 + q, 0), g.NX - 1) * g.NY + cj));
     }
     if (any_xh) {
-        const float* psi = choose(xhigh, pp.psi_h[0][1], pp.psi_h[0][0]) + (long long)s * fxh.p * g.NY;
+        const float* psi = choose(xhigh, pp.psi_h[par][1], pp.psi_h[par][0]) + (long long)s * fxh.p * g.NY;
 #pragma unroll
         for (int q = 0; q < KR; ++q) pxh[q] = ld(psi, 4u * (unsigned)(fxh.at(i0 + q) * g.NY + cj));
     }
     if (any_xe) {
-        const float* psi = choose(xhigh, pp.psi_e[0][1], pp.psi_e[0][0]) + (long long)s * (fxe.p + 1) * g.NY;
+        const float* psi = choose(xhigh, pp.psi_e[par][1], pp.psi_e[par][0]) + (long long)s * (fxe.p + 1) * g.NY;
 #pragma unroll
         for (int q = 0; q < KR; ++q) pxe[q] = ld(psi, 4u * (unsigned)(fxe.at(i0 + q) * g.NY + cj));
     }
     if (yh) {
-        const float* psi = choose(yhigh, pp.psi_h[0][3], pp.psi_h[0][2]) + (long long)s * g.NX * fyh.p + fyh.at(gj);
+        const float* psi = choose(yhigh, pp.psi_h[par][3], pp.psi_h[par][2]) + (long long)s * g.NX * fyh.p + fyh.at(gj);
 #pragma unroll
         for (int q = 0; q < KR; ++q) pyh[q] = psi[min(max(i0 + q, 0), g.NX - 1) * fyh.p];
         cyh = cpml_profile(choose(yhigh, f.coef_h[3], f.coef_h[2]), fyh.p, fyh.at(gj));
     }
     if (ye) {
         const int depth = fye.p + 1;
-        const float* psi = choose(yhigh, pp.psi_e[0][3], pp.psi_e[0][2]) + (long long)s * g.NX * depth + fye.at(gj);
+        const float* psi = choose(yhigh, pp.psi_e[par][3], pp.psi_e[par][2]) + (long long)s * g.NX * depth + fye.at(gj);
 #pragma unroll
         for (int q = 0; q < KR; ++q) pye[q] = psi[min(max(i0 + q, 0), g.NX - 1) * depth];
         cye = cpml_profile(choose(yhigh, f.coef_e[3], f.coef_e[2]), fye.p, fye.at(gj));
@@ -324,13 +316,13 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
         o[3] = c.rf;
     }
     int sbeg = 0, send = 0, rbeg = 0, rend = 0;
-    if (args.src.count > 0) {
-        sbeg = args.src.block_off[lt];
-        send = args.src.block_off[lt + 1];
+    if (args->src.count > 0) {
+        sbeg = args->src.block_off[lt];
+        send = args->src.block_off[lt + 1];
     }
-    if (args.rx.count > 0) {
-        rbeg = args.rx.off[lt];
-        rend = args.rx.off[lt + 1];
+    if (args->rx.count > 0) {
+        rbeg = args->rx.off[lt];
+        rend = args->rx.off[lt + 1];
     }
     // conditions of the strip's rows, one bit each
     const unsigned m_in = row_range(i0, KR, 1, g.NX - 2);  // Hx and Ez updated
@@ -344,7 +336,7 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
     const bool box_col = own_col && gj >= hist.box.y0 && gj < hist.box.y0 + hist.box.ny;
     const bool listed = rend > rbeg;
     const bool save = hist.on;
-    int frame = args.frame, next = frame * hist.S;  // the next saved step
+    int next = frame * hist.S;  // the next saved step
     for (int sub = 0; sub < nsub; ++sub) {
         const int it = it0 + sub;
         // magnetic half step
@@ -403,7 +395,7 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
             exchange<KR, NW, UP, DN>(hy, h_first, h_last, w, lane, h);
             if (listed) {
                 if (sub > 0) {  // receivers of the step before: every row of s_ez is there since the first barrier
-                    const auto& rx = args_now()->rx;
+                    const auto& rx = again(args)->rx;
                     for (int x = rbeg + (int)threadIdx.x; x < rend; x += NW * 64) {
                         const int2 ent = rx.ent[x];
                         rx.out[((long long)s * rx.nt + it - 1) * rx.nrx + ent.y] = s_ez[ent.x];
@@ -454,7 +446,7 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
                 }
             }
             for (int x = sbeg; x < send; ++x) {
-                const auto& src = args_now()->src;
+                const auto& src = again(args)->src;
                 const int2 ent = src.entries[x];
                 const int row = ent.x >> 6;
                 if (row / KR != w) continue;
@@ -464,7 +456,7 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
                     if (row - w * KR == q && (ent.x & 63) == lane) ez[q] -= cb[q] * scale;
             }
             if (save && it == next) {
-                const auto& hist = args_now()->hist;
+                const auto& hist = again(args)->hist;
                 const unsigned br = rows_now(m_box), ur = rows_now(m_in);
                 const int comps = hist.mode == 3 ? 3 : 1;
                 const int ny = hist.box.ny;
@@ -508,7 +500,7 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
     }
     if (rend > rbeg) {
         __syncthreads();
-        const auto& rx = args_now()->rx;
+        const auto& rx = again(args)->rx;
         for (int x = rbeg + (int)threadIdx.x; x < rend; x += NW * 64) {
             const int2 ent = rx.ent[x];
             rx.out[((long long)s * rx.nt + it0 + nsub - 1) * rx.nrx + ent.y] = s_ez[ent.x];
@@ -519,9 +511,9 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
     asm volatile("" : "+s"(ib), "+v"(jb));
     if (!own_col) return;
     {
-    const auto& pp = args_now()->pp;
-    const auto& g = args_now()->g;
-    float *oez = pp.Ez[1] + sb, *ohx = pp.Hx[1] + sb, *ohy = pp.Hy[1] + sb;
+    const auto& pp = again(args)->pp;
+    const auto& g = again(args)->g;
+    float *oez = pp.Ez[par ^ 1] + sb, *ohx = pp.Hx[par ^ 1] + sb, *ohy = pp.Hy[par ^ 1] + sb;
 #pragma unroll
     for (int q = 0; q < KR; ++q) {
         if (!row_of(m_own, q)) continue;
@@ -531,31 +523,38 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
         put(ohy, p, hy[q]);
     }
     if (any_xh) {
-        float* psi = choose(xhigh, pp.psi_h[1][1], pp.psi_h[1][0]) + (long long)s * fxh.p * g.NY;
+        float* psi = choose(xhigh, pp.psi_h[par ^ 1][1], pp.psi_h[par ^ 1][0]) + (long long)s * fxh.p * g.NY;
 #pragma unroll
         for (int q = 0; q < KR; ++q)
             if (row_of(m_own & m_xh, q)) put(psi, 4u * (unsigned)(fxh.at(ib + q) * g.NY + jb), pxh[q]);
     }
     if (any_xe) {
-        float* psi = choose(xhigh, pp.psi_e[1][1], pp.psi_e[1][0]) + (long long)s * (fxe.p + 1) * g.NY;
+        float* psi = choose(xhigh, pp.psi_e[par ^ 1][1], pp.psi_e[par ^ 1][0]) + (long long)s * (fxe.p + 1) * g.NY;
 #pragma unroll
         for (int q = 0; q < KR; ++q)
             if (row_of(m_own & m_xe, q)) put(psi, 4u * (unsigned)(fxe.at(ib + q) * g.NY + jb), pxe[q]);
     }
     if (yh) {
-        float* psi = choose(yhigh, pp.psi_h[1][3], pp.psi_h[1][2]) + (long long)s * g.NX * fyh.p + fyh.at(jb);
+        float* psi = choose(yhigh, pp.psi_h[par ^ 1][3], pp.psi_h[par ^ 1][2]) + (long long)s * g.NX * fyh.p + fyh.at(jb);
 #pragma unroll
         for (int q = 0; q < KR; ++q)
             if (row_of(m_own, q)) psi[(ib + q) * fyh.p] = pyh[q];
     }
     if (ye) {
         const int depth = fye.p + 1;
-        float* psi = choose(yhigh, pp.psi_e[1][3], pp.psi_e[1][2]) + (long long)s * g.NX * depth + fye.at(jb);
+        float* psi = choose(yhigh, pp.psi_e[par ^ 1][3], pp.psi_e[par ^ 1][2]) + (long long)s * g.NX * depth + fye.at(jb);
 #pragma unroll
         for (int q = 0; q < KR; ++q)
             if (row_of(m_own, q)) psi[(ib + q) * depth] = pye[q];
     }
     }
+}
+
+template <int ORDER, int KR, int NW, int T>
+__global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs a)
+{
+    strip_fwd<ORDER, KR, NW, T>((StripArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(), blockIdx.y, blockIdx.x,
+                                blockIdx.z, a.it0, a.nsub, a.frame, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -574,25 +573,6 @@ __global__ __launch_bounds__(NW * 64) void k_tm_strip_fwd(StripArgs args)
 // in its own rows of s_lz. The material terms of a saved step go to one buffer
 // a saved step of the launch (summed over shots afterwards) or, with DIRECT (one
 // shot), into the sums themselves, which the launch keeps in registers.
-struct StripAdjArgs {
-    Tm2dGrid g;
-    Tm2dFields f;
-    TmPingPong pp;
-    StripMap sm;
-    SourceBlocks src;
-    TmReceiversAdj rx;
-    StripGrad mg;
-    float inv[2];
-    int it0, nsub, frame;  // steps it0 .. it0 - nsub + 1, the newest saved step's frame
-};
-typedef const __attribute__((address_space(4))) StripAdjArgs* StripAdjArgsPtr;
-__device__ __forceinline__ StripAdjArgsPtr adj_args_now()
-{
-    StripAdjArgsPtr a = (StripAdjArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(a));
-    return a;
-}
-
 // LDS of one wavefront is read in the order it was written; this keeps the
 // compiler to it where lanes read what other lanes wrote.
 __device__ __forceinline__ void wave_lds_order()
@@ -601,17 +581,26 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_wave_barrier();
 }
 
+// Tile (ti, tj) of shot s, steps it0 .. it0 - nsub + 1; ts: the newest saved
+// step's frame.
+// += in the cache, without waiting for the value: one rounded addition, in order
+// with this thread's earlier ones to the same address.
+__device__ __forceinline__ void add_owned(double* p, double v)
+{
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void add_owned(float* p, float v) { *p += v; }
+
 template <int ORDER, int KR, int NW, int T, bool DIRECT, typename ACC>
-__global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip_adj(StripAdjArgs args)
+__device__ __forceinline__ void strip_adj(StripAdjArgsPtr args, int ti, int tj, int s, int it0, int nsub, int ts,
+                                          int par)
 {
     using St = Strip<ORDER, KR, NW, T>;
     constexpr int R = St::R, H = St::H, SR = St::SR;
-    const Tm2dGrid& g = args.g;
-    const Tm2dFields& f = args.f;
-    const TmPingPong& pp = args.pp;
-    const StripMap& sm = args.sm;
-    const int it0 = args.it0, nsub = args.nsub;
-    const int tj = blockIdx.x, ti = blockIdx.y, s = blockIdx.z;
+    const auto& g = args->g;
+    const auto& f = args->f;
+    const auto& pp = args->pp;
+    const auto& sm = args->sm;
     const int tile = ti * sm.ntj + tj;
     __shared__ float e_first[NW][R][64], e_last[NW][R > 1 ? R - 1 : 1][64];
     __shared__ float h_first[NW][R > 1 ? R - 1 : 1][64], h_last[NW][R][64];
@@ -632,7 +621,7 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
 
     float lz[KR], lx[KR], ly[KR], ca[KR], cc[KR], cb[KR], hc[KR], hr[KR];
     float pxe[KR], pye[KR], pxh[KR], pyh[KR];
-    const float *gez = pp.Ez[0] + sb, *ghx = pp.Hx[0] + sb, *ghy = pp.Hy[0] + sb;
+    const float *gez = pp.Ez[par] + sb, *ghx = pp.Hx[par] + sb, *ghy = pp.Hy[par] + sb;
 #pragma unroll
     for (int q = 0; q < KR; ++q) {
         const unsigned p = 4u * (unsigned)(min(max(i0 + q, 0), g.NX - 1) * g.NY + cj);
@@ -656,17 +645,17 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
         for (int q = 0; q < KR; ++q) hr[q] = ld(f.hrhs, 4u * (unsigned)(min(max(i0 + q, 0), g.NX - 1) * g.NY + cj));
     }
     if (any_xh) {
-        const float* psi = choose(xhigh, pp.psi_h[0][1], pp.psi_h[0][0]) + (long long)s * fxh.p * g.NY;
+        const float* psi = choose(xhigh, pp.psi_h[par][1], pp.psi_h[par][0]) + (long long)s * fxh.p * g.NY;
 #pragma unroll
         for (int q = 0; q < KR; ++q) pxh[q] = ld(psi, 4u * (unsigned)(fxh.at(i0 + q) * g.NY + cj));
     }
     if (any_xe) {
-        const float* psi = choose(xhigh, pp.psi_e[0][1], pp.psi_e[0][0]) + (long long)s * (fxe.p + 1) * g.NY;
+        const float* psi = choose(xhigh, pp.psi_e[par][1], pp.psi_e[par][0]) + (long long)s * (fxe.p + 1) * g.NY;
 #pragma unroll
         for (int q = 0; q < KR; ++q) pxe[q] = ld(psi, 4u * (unsigned)(fxe.at(i0 + q) * g.NY + cj));
     }
     if (yh) {
-        const float* psi = choose(yhigh, pp.psi_h[0][3], pp.psi_h[0][2]) + (long long)s * g.NX * fyh.p + fyh.at(gj);
+        const float* psi = choose(yhigh, pp.psi_h[par][3], pp.psi_h[par][2]) + (long long)s * g.NX * fyh.p + fyh.at(gj);
 #pragma unroll
         for (int q = 0; q < KR; ++q) pyh[q] = psi[min(max(i0 + q, 0), g.NX - 1) * fyh.p];
         if (w == 0) {
@@ -676,7 +665,7 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
     }
     if (ye) {
         const int depth = fye.p + 1;
-        const float* psi = choose(yhigh, pp.psi_e[0][3], pp.psi_e[0][2]) + (long long)s * g.NX * depth + fye.at(gj);
+        const float* psi = choose(yhigh, pp.psi_e[par][3], pp.psi_e[par][2]) + (long long)s * g.NX * depth + fye.at(gj);
 #pragma unroll
         for (int q = 0; q < KR; ++q) pye[q] = psi[min(max(i0 + q, 0), g.NX - 1) * depth];
         if (w == 0) {
@@ -698,26 +687,26 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
         o[2] = c.re;
         o[3] = c.rf;
     }
-    const float invx = args.inv[0], invy = args.inv[1];
+    const float invx = args->inv[0], invy = args->inv[1];
     int sbeg = 0, send = 0, rbeg = 0, rend = 0;
-    if (args.src.count > 0) {
-        sbeg = args.src.block_off[lt];
-        send = args.src.block_off[lt + 1];
+    if (args->src.count > 0) {
+        sbeg = args->src.block_off[lt];
+        send = args->src.block_off[lt + 1];
     }
-    if (args.rx.count > 0) {
-        rbeg = args.rx.off[lt];
-        rend = args.rx.off[lt + 1];
+    if (args->rx.count > 0) {
+        rbeg = args->rx.off[lt];
+        rend = args->rx.off[lt + 1];
     }
     // the first 64 receiver cells of the tile: a lane's own one, its data a step ahead
     int4 mine = make_int4(-1, 0, 0, 0);
     int first = 0;
     float ahead = 0.0f;
     if (rbeg + lane < rend) {
-        const int4 e = args.rx.grp[rbeg + lane];
+        const int4 e = args->rx.grp[rbeg + lane];
         if ((e.x >> 6) / KR == w) {
             mine = e;
-            first = args.rx.member[e.y];
-            ahead = args.rx.dgrad[((long long)s * args.rx.nt + it0) * args.rx.nrx + first];
+            first = args->rx.member[e.y];
+            ahead = args->rx.dgrad[((long long)s * args->rx.nt + it0) * args->rx.nrx + first];
         }
     }
     const bool any_rx = __any(mine.x >= 0) || rend - rbeg > 64;
@@ -733,29 +722,32 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
     const bool hx_col = gj >= 0 && gj < g.NY - 1;
 
     // material terms: factors of each cell (none: all zero), the sums of one shot
-    const Box& box = args.mg.box;
-    const bool mat = args.mg.on;
+    const auto& box = args->mg.box;
+    const bool mat = args->mg.on;
     const unsigned m_box = mat ? m_own & row_range(i0, KR, box.x0, box.x0 + box.nx - 1) : 0u;
     const bool box_col = own_col && gj >= box.y0 && gj < box.y0 + box.ny;
     unsigned active = 0;
-    ACC ge[DIRECT ? KR : 1], gs[DIRECT ? KR : 1];
-    const int S = args.mg.S;
-    int ts = args.frame, next = mat ? ts * S : -1;
+    // FP64 sums of four rows would be 16 registers: they are added in memory, by
+    // the one thread that owns the cell
+    constexpr bool ATOMIC = DIRECT && KR > 2 && sizeof(ACC) == 8, REGS = DIRECT && !ATOMIC;
+    ACC ge[REGS ? KR : 1], gs[REGS ? KR : 1];
+    const int S = args->mg.S;
+    int next = mat ? ts * S : -1;
     if (mat) {
-        const float dt = args.mg.dt;
+        const float dt = args->mg.dt;
 #pragma unroll
         for (int q = 0; q < KR; ++q) {
             if (!row_of(m_box, q) || !box_col) continue;
             const int gi = i0 + q;
-            const float sig = args.mg.sig[(long long)gi * g.NY * 2 + (long long)gj * 2];  // full-layout material index
+            const float sig = args->mg.sig[(long long)gi * g.NY * 2 + (long long)gj * 2];  // full-layout material index
             active |= sig <= kPecSigma ? 1u << q : 0u;
             s_mat[(w * KR + q) * 64 + lane] =
                 make_float4(kEps0 * (1.0f - ca[q]) * cb[q] / dt, -kEps0 * cb[q] * cb[q] / dt,
                             -0.5f * (1.0f + ca[q]) * cb[q], -0.5f * cb[q] * cb[q]);
-            if constexpr (DIRECT) {
+            if constexpr (REGS) {
                 const long long o = (long long)gi * (g.NY - 1) + gj;
-                ge[q] = args.mg.want_eps ? ((const ACC*)args.mg.geps)[o] : (ACC)0;
-                gs[q] = args.mg.want_sig ? ((const ACC*)args.mg.gsig)[o] : (ACC)0;
+                ge[q] = args->mg.want_eps ? ((const ACC*)args->mg.geps)[o] : (ACC)0;
+                gs[q] = args->mg.want_sig ? ((const ACC*)args->mg.gsig)[o] : (ACC)0;
             }
         }
     }
@@ -767,7 +759,7 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
         const bool save = it == next;
         float m_e[KR], m_s[KR];
         if (save && m_box) {
-            const auto& mg = adj_args_now()->mg;
+            const auto& mg = again(args)->mg;
             const int ny = mg.box.ny;
             const unsigned at = (unsigned)((i0 - mg.box.x0) * ny + (gj - mg.box.y0));
             const bool last = mg.e_only && ts + 1 >= mg.nt_saved;
@@ -791,7 +783,7 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
         }
         // receivers^T
         if (any_rx) {
-            const auto& rx = adj_args_now()->rx;
+            const auto& rx = again(args)->rx;
 #pragma unroll
             for (int q = 0; q < KR; ++q) s_lz[(w * KR + q) * 64 + lane] = lz[q];
             wave_lds_order();
@@ -815,7 +807,7 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
         }
         // source^T: one value per (step, shot, source), summed over shots later
         for (int x = sbeg; x < send; ++x) {
-            const auto& a = *adj_args_now();
+            const auto& a = *again(args);
             const int2 ent = a.src.entries[x];
             const int row = ent.x >> 6;
             if (row / KR != w) continue;
@@ -917,7 +909,7 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
             exchange<KR, NW, UP, DN>(vx, h_first, h_last, w, lane, h);
             // the material terms here: the history's loads had the half steps to arrive
             if (save && m_box) {
-                const auto& mg = adj_args_now()->mg;
+                const auto& mg = again(args)->mg;
                 const float wgt = (float)min(S, mg.nt - it);
                 const int ny = mg.box.ny;
                 const unsigned at = 4u * (unsigned)((i0 - mg.box.x0) * ny + (gj - mg.box.y0));
@@ -940,15 +932,18 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
                     const float gca = up ? l * m_e[q] * wgt : 0.0f;
                     const float gcb = l * rhs * wgt;
                     const bool on = (active >> q) & 1u;
+                    const long long o = (long long)(i0 + q) * (g.NY - 1) + gj;
                     const float4 d = s_mat[(w * KR + q) * 64 + lane];
                     if (mg.want_eps) {
                         const float t = on ? gca * d.x + gcb * d.y : 0.0f;
-                        if constexpr (DIRECT) ge[q] += (ACC)0 + (ACC)t;
+                        if constexpr (REGS) ge[q] += (ACC)0 + (ACC)t;
+                        else if constexpr (ATOMIC) add_owned((ACC*)mg.geps + o, (ACC)0 + (ACC)t);
                         else put(te, at + 4u * (unsigned)(q * ny), t);
                     }
                     if (mg.want_sig) {
                         const float t = on ? gca * d.z + gcb * d.w : 0.0f;
-                        if constexpr (DIRECT) gs[q] += (ACC)0 + (ACC)t;
+                        if constexpr (REGS) gs[q] += (ACC)0 + (ACC)t;
+                        else if constexpr (ATOMIC) add_owned((ACC*)mg.gsig + o, (ACC)0 + (ACC)t);
                         else put(ts1, at + 4u * (unsigned)(q * ny), t);
                     }
                 }
@@ -990,9 +985,9 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
     asm volatile("" : "+s"(ib), "+v"(jb));
     if (!own_col) return;
     {
-        const auto& pp = adj_args_now()->pp;
-        const auto& g = adj_args_now()->g;
-        float *oez = pp.Ez[1] + sb, *ohx = pp.Hx[1] + sb, *ohy = pp.Hy[1] + sb;
+        const auto& pp = again(args)->pp;
+        const auto& g = again(args)->g;
+        float *oez = pp.Ez[par ^ 1] + sb, *ohx = pp.Hx[par ^ 1] + sb, *ohy = pp.Hy[par ^ 1] + sb;
 #pragma unroll
         for (int q = 0; q < KR; ++q) {
             if (!row_of(m_own, q)) continue;
@@ -1001,8 +996,8 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
             put(ohx, p, lx[q]);
             put(ohy, p, ly[q]);
         }
-        if constexpr (DIRECT) {
-            const auto& mg = adj_args_now()->mg;
+        if constexpr (REGS) {
+            const auto& mg = again(args)->mg;
             if (box_col) {
 #pragma unroll
                 for (int q = 0; q < KR; ++q) {
@@ -1014,31 +1009,38 @@ __global__ __launch_bounds__(NW * 64, DIRECT && NW == 8 ? 2 : 4) void k_tm_strip
             }
         }
         if (any_xh) {
-            float* psi = choose(xhigh, pp.psi_h[1][1], pp.psi_h[1][0]) + (long long)s * fxh.p * g.NY;
+            float* psi = choose(xhigh, pp.psi_h[par ^ 1][1], pp.psi_h[par ^ 1][0]) + (long long)s * fxh.p * g.NY;
 #pragma unroll
             for (int q = 0; q < KR; ++q)
                 if (row_of(m_own & m_xh, q)) put(psi, 4u * (unsigned)(fxh.at(ib + q) * g.NY + jb), pxh[q]);
         }
         if (any_xe) {
-            float* psi = choose(xhigh, pp.psi_e[1][1], pp.psi_e[1][0]) + (long long)s * (fxe.p + 1) * g.NY;
+            float* psi = choose(xhigh, pp.psi_e[par ^ 1][1], pp.psi_e[par ^ 1][0]) + (long long)s * (fxe.p + 1) * g.NY;
 #pragma unroll
             for (int q = 0; q < KR; ++q)
                 if (row_of(m_own & m_xe, q)) put(psi, 4u * (unsigned)(fxe.at(ib + q) * g.NY + jb), pxe[q]);
         }
         if (yh) {
-            float* psi = choose(yhigh, pp.psi_h[1][3], pp.psi_h[1][2]) + (long long)s * g.NX * fyh.p + fyh.at(jb);
+            float* psi = choose(yhigh, pp.psi_h[par ^ 1][3], pp.psi_h[par ^ 1][2]) + (long long)s * g.NX * fyh.p + fyh.at(jb);
 #pragma unroll
             for (int q = 0; q < KR; ++q)
                 if (row_of(m_own, q)) psi[(ib + q) * fyh.p] = pyh[q];
         }
         if (ye) {
             const int depth = fye.p + 1;
-            float* psi = choose(yhigh, pp.psi_e[1][3], pp.psi_e[1][2]) + (long long)s * g.NX * depth + fye.at(jb);
+            float* psi = choose(yhigh, pp.psi_e[par ^ 1][3], pp.psi_e[par ^ 1][2]) + (long long)s * g.NX * depth + fye.at(jb);
 #pragma unroll
             for (int q = 0; q < KR; ++q)
                 if (row_of(m_own, q)) psi[(ib + q) * depth] = pye[q];
         }
     }
+}
+
+template <int ORDER, int KR, int NW, int T, bool DIRECT, typename ACC>
+__global__ __launch_bounds__(NW * 64, 4) void k_tm_strip_adj(StripAdjArgs a)
+{
+    strip_adj<ORDER, KR, NW, T, DIRECT, ACC>((StripAdjArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(), blockIdx.y,
+                                             blockIdx.x, blockIdx.z, a.it0, a.nsub, a.frame, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1066,8 +1068,7 @@ namespace {
 // Hence the rule of map_order: shape 0 as long as each of its workgroups (1024
 // threads) has a compute unit to itself, shape 1 as long as its workgroups (512
 // threads, two a compute unit) are all resident at once, then shape 2, whose
-// larger tile has the smaller margin; one shot stays at shape 1, since the sums
-// of its material gradients in registers would make shape 2 spill.
+// larger tile has the smaller margin.
 template <int ORDER, int SIZE>
 struct Shapes;
 template <>
@@ -1119,7 +1120,7 @@ StripMap map_order(const Tm2dGrid& g)
     const StripMap small = make_strip_map(shape_of<ORDER, 0>(), g.NX, g.NY);
     if ((long long)small.tiles * g.nshot <= 256) return small;
     const StripMap mid = make_strip_map(shape_of<ORDER, 1>(), g.NX, g.NY);
-    if (g.nshot == 1 || (long long)mid.tiles * g.nshot <= 512) return mid;
+    if ((long long)mid.tiles * g.nshot <= 512) return mid;
     return make_strip_map(shape_of<ORDER, 2>(), g.NX, g.NY);
 }
 }  // namespace
@@ -1152,9 +1153,7 @@ void launch_adj_shape(const dim3& grid, const StripAdjArgs& a, bool fp64, hipStr
     constexpr int KR = P::KR, NW = P::NW, T = P::T;
     const dim3 block(NW * 64);
     const bool direct = a.mg.on && a.g.nshot == 1;
-    if (SIZE == 2 || !direct)
-        hipLaunchKernelGGL((k_tm_strip_adj<ORDER, KR, NW, T, false, float>), grid, block, 0, st, a);
-    else if constexpr (SIZE == 2) return;  // several shots, see map_order
+    if (!direct) hipLaunchKernelGGL((k_tm_strip_adj<ORDER, KR, NW, T, false, float>), grid, block, 0, st, a);
     else if (fp64) hipLaunchKernelGGL((k_tm_strip_adj<ORDER, KR, NW, T, true, double>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((k_tm_strip_adj<ORDER, KR, NW, T, true, float>), grid, block, 0, st, a);
 }
@@ -1175,6 +1174,82 @@ void launch_tm_strip_adj(int order, const Tm2dGrid& g, const Tm2dFields& f, cons
     const StripAdjArgs a{g, f, pp, sm, src, rx, mg, {1.0f / g.d[0], 1.0f / g.d[1]}, it0, nsub,
                           it0 / std::max(mg.S, 1)};
     order == 4 ? launch_adj_order<4>(grid, a, fp64, st) : launch_adj_order<2>(grid, a, fp64, st);
+}
+
+// ---------------------------------------------------------------------------
+// Batches: one launch advances every one-shot instance of one order and phase
+// ---------------------------------------------------------------------------
+// A batch fills the chip with its instances, so they take shape 2. Twelve
+// gradients of 148 to 404 cells a side, orders 2 and 4 by halves: a step of the
+// one-step kernels takes 12 (forward) and 24 us (adjoint) at order 4, 10 and 21
+// at order 2, one launch after the other; these take 15.7 us for 2 steps of both
+// phases at order 4 and 27 for 6 at order 2. With a launch a phase each took
+// 14 to 16 and 23 to 27.
+namespace {
+template <int ORDER>
+using BatchShape = Shapes<ORDER, 2>;
+
+// Instance of workgroup b by bisection of the prefix sums; b becomes its tile.
+__device__ __forceinline__ int batch_instance(const int* __restrict__ prefix, int ninst, int& b)
+{
+    int lo = 0, hi = ninst - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (prefix[mid] <= b) lo = mid;
+        else hi = mid - 1;
+    }
+    const int k = __builtin_amdgcn_readfirstlane(lo);
+    b = __builtin_amdgcn_readfirstlane(b - prefix[k]);
+    return k;
+}
+
+// Both phases in one launch, adjoint workgroups (the longer ones) first:
+// apart, each left half of the compute units idle.
+template <int ORDER>
+__global__ __launch_bounds__(BatchShape<ORDER>::NW * 64, 4) void k_tm_strip_batch(StripBatchSlot fwd,
+                                                                                  StripBatchSlot adj, int gstep,
+                                                                                  int launch, int nsub)
+{
+    using P = BatchShape<ORDER>;
+    // XCD x takes the x-th contiguous chunk of workgroups
+    int b = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
+    if (b < adj.total) {
+        const int k = batch_instance(adj.prefix, adj.ninst, b);
+        const StripBatchInst& I = adj.insts[k];
+        const int ti = b / I.adj.sm.ntj, it0 = I.nt - 1 - (gstep - I.start);
+        strip_adj<ORDER, P::KR, P::NW, P::T, true, double>((StripAdjArgsPtr)&I.adj, ti, b - ti * I.adj.sm.ntj, 0, it0,
+                                                           nsub, it0, (launch - I.launch) & 1);
+    } else {
+        b -= adj.total;
+        if (b >= fwd.total) return;
+        const int k = batch_instance(fwd.prefix, fwd.ninst, b);
+        const StripBatchInst& I = fwd.insts[k];
+        const int ti = b / I.fwd.sm.ntj, it0 = gstep - I.start;
+        strip_fwd<ORDER, P::KR, P::NW, P::T>((StripArgsPtr)&I.fwd, ti, b - ti * I.fwd.sm.ntj, 0, it0, nsub, it0,
+                                             (launch - I.launch) & 1);
+    }
+}
+}  // namespace
+
+StripMap strip_batch_map(int order, const Tm2dGrid& g)
+{
+    return make_strip_map(order == 4 ? shape_of<4, 2>() : shape_of<2, 2>(), g.NX, g.NY);
+}
+
+int strip_batch_steps(int order) { return order == 4 ? BatchShape<4>::T : BatchShape<2>::T; }
+
+void launch_tm_strip_batch(int order, const StripBatchSlot& fwd, const StripBatchSlot& adj, int gstep, int launch,
+                           int nsub, hipStream_t st)
+{
+    const int total = fwd.total + adj.total;
+    if (total <= 0) return;
+    const dim3 grid((unsigned)((total + 7) / 8 * 8));
+    if (order == 4)
+        hipLaunchKernelGGL(k_tm_strip_batch<4>, grid, dim3(BatchShape<4>::NW * 64), 0, st, fwd, adj, gstep, launch,
+                           nsub);
+    else
+        hipLaunchKernelGGL(k_tm_strip_batch<2>, grid, dim3(BatchShape<2>::NW * 64), 0, st, fwd, adj, gstep, launch,
+                           nsub);
 }
 
 }  // namespace dgx

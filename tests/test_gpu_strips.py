@@ -7,6 +7,7 @@ PEC cells, every history that the 2D path keeps, and sources and coincident
 receivers in margins, on tile corners, in the CPML and on the grid's edges."""
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +76,51 @@ def test_strips_match_oracle_bitwise(oracle_built, cuda_device, monkeypatch, cas
         assert np.array_equal(gpu["L"][k], cpu["L"][k]), k
     assert np.array_equal(gpu["E_saved"], cpu["E_saved"])
     assert np.array_equal(gpu["R_saved"], cpu["R_saved"])
+
+
+def _request(rid, shape, nt, order, nshot, gradient, seed):
+    from deepgpr_amd.serving import SolveRequest
+    gen = torch.Generator().manual_seed(seed)
+    eps = 1.0 + 8.0 * torch.rand(shape, generator=gen)
+    sig = 0.01 * torch.rand(shape, generator=gen)
+    t = torch.arange(nt, dtype=torch.float32) * 3e-11
+    a2 = (torch.pi * 4e8 * (t - 2.5e-9)) ** 2
+    wave = ((1 - 2 * a2) * torch.exp(-a2)).reshape(1, nt, 1)
+    src = torch.tensor([[[shape[0] // 2 - s, shape[1] // 2, 0]] for s in range(nshot)])
+    rx = torch.tensor([[[5 + 3 * (r % 4), 2 + 5 * r, 0] for r in range(9)] for _ in range(nshot)])
+    return SolveRequest(eps, sig, wave, src, rx, 0.02, 3e-11, fdtd_order=order, pmlthick=8, gradient=gradient,
+                        rid=rid, options={"mode": 2, "wavefield_rhs_history": "reconstructed",
+                                              "wavefield_storage_dtype": torch.bfloat16 if rid % 3 == 1
+                                              else torch.float32})
+
+
+def test_batch_of_strips_equals_one_step_launches(cuda_device, monkeypatch):
+    """Instances that run several steps a launch beside some that cannot (order
+    8, two shots), in both phases at once and with steps that end inside a
+    launch: the bits of the same solves one at a time, one step a launch."""
+    from deepgpr_amd import batch, serving
+    shapes = [(60, 52), (91, 77), (52, 104), (110, 47), (48, 48), (75, 130)]
+    reqs = [_request(k, shapes[k % 6], 37 + 8 * (k % 5), (2, 4, 4, 2, 8, 4, 2)[k % 7], 2 if k % 6 == 5 else 1,
+                     k % 4 != 3, 900 + k) for k in range(13)]
+    monkeypatch.setenv("DEEPGPR_AMD_TM2D_STRIPS", "0")
+    alone = serving.run_sequential(reqs, cuda_device)["results"]
+
+    def batched(strips):
+        monkeypatch.setenv("DEEPGPR_AMD_TM2D_STRIPS", strips)
+        with batch.BatchSolver(cuda_device) as solver:
+            ids = {solver.add(r): r.rid for r in reqs[:7]}
+            solver.step(40)  # joins while some are in their adjoint
+            ids.update({solver.add(r): r.rid for r in reqs[7:]})
+            solver.run(11)
+            return {ids[n]: solver.result(n) for n in ids}
+
+    for strips in ("1", "0"):
+        print(f"[gpu strips] batch, strips {strips}", flush=True)
+        got = batched(strips)
+        for r in reqs:
+            a = alone[r.rid]
+            res = got[r.rid]
+            assert torch.equal(res[0], a.receivers), (strips, r.rid)
+            if r.gradient:
+                assert torch.equal(res[1], a.grad_eps_r), (strips, r.rid)
+                assert torch.equal(res[2], a.grad_sigma), (strips, r.rid)
