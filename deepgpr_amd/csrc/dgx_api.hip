@@ -639,7 +639,9 @@ int tm2d_probe(const Plan& pl, const dgx_solve* P, hipStream_t stream, double* u
     float* co = b + 6 * field;
     const float* full[5] = {P->update_coeff[0], P->update_coeff[1], P->update_coeff[2], P->update_coeff[4],
                             P->update_coeff[5]};
-    for (int c = 0; c < 5; ++c) launch_tm_pack(full[c], co + (long long)c * g0.plane, g0.plane, false, stream);
+    TmMoves mv{};
+    for (int c = 0; c < 5; ++c) mv.add(kTmPack, full[c], co + (long long)c * g0.plane, g0.plane);
+    launch_tm_moves(mv, stream);
     f.Ez = pp.Ez[0];
     f.Hx = pp.Hx[0];
     f.Hy = pp.Hy[0];
@@ -775,7 +777,8 @@ struct Tm2dState {
         float* co = b + nf * field;
         const float* full[5] = {P->update_coeff[0], P->update_coeff[1], P->update_coeff[2], P->update_coeff[4],
                                 P->update_coeff[5]};
-        for (int c = 0; c < 5; ++c) launch_tm_pack(full[c], co + (long long)c * g.plane, g.plane, false, stream);
+        TmMoves mv{};  // 8 planes and, fused, up to 8 auxiliaries
+        for (int c = 0; c < 5; ++c) mv.add(kTmPack, full[c], co + (long long)c * g.plane, g.plane);
         f.ca = co;
         f.ccurl = co + g.plane;
         f.cb = co + 2 * (long long)g.plane;
@@ -794,10 +797,13 @@ struct Tm2dState {
             psi_len_h[f4] = g.pml[f4] > 0 ? across * g.pml[f4] : 0;
             alt_len += psi_len_e[f4] + psi_len_h[f4];
         }
-        launch_tm_pack(P->E[2], f.Ez, field, false, stream);
-        launch_tm_pack(P->H[0], f.Hx, field, false, stream);
-        launch_tm_pack(P->H[1], f.Hy, field, false, stream);
-        if (!fused) return 0;
+        mv.add(kTmPack, P->E[2], f.Ez, field);
+        mv.add(kTmPack, P->H[0], f.Hx, field);
+        mv.add(kTmPack, P->H[1], f.Hy, field);
+        if (!fused) {
+            launch_tm_moves(mv, stream);
+            return 0;
+        }
         pp.Ez[0] = f.Ez;
         pp.Hx[0] = f.Hx;
         pp.Hy[0] = f.Hy;
@@ -812,16 +818,13 @@ struct Tm2dState {
             pp.psi_e[0][f4] = home_e[f4];
             pp.psi_h[0][f4] = home_h[f4];
             pp.psi_e[1][f4] = psi_len_e[f4] ? a : nullptr;
-            if (psi_len_e[f4] &&
-                hipMemcpyAsync(a, home_e[f4], psi_len_e[f4] * 4, hipMemcpyDeviceToDevice, stream) != hipSuccess)
-                return -1;
+            mv.add(kTmCopy, home_e[f4], a, psi_len_e[f4]);
             a += psi_len_e[f4];
             pp.psi_h[1][f4] = psi_len_h[f4] ? a : nullptr;
-            if (psi_len_h[f4] &&
-                hipMemcpyAsync(a, home_h[f4], psi_len_h[f4] * 4, hipMemcpyDeviceToDevice, stream) != hipSuccess)
-                return -1;
+            mv.add(kTmCopy, home_h[f4], a, psi_len_h[f4]);
             a += psi_len_h[f4];
         }
+        launch_tm_moves(mv, stream);
         return 0;
     }
     // after a fused step: what was written becomes what is read
@@ -835,27 +838,21 @@ struct Tm2dState {
             std::swap(pp.psi_h[0][f4], pp.psi_h[1][f4]);
         }
     }
-    int unpack(const dgx_solve* P, hipStream_t stream)
+    void unpack(const dgx_solve* P, hipStream_t stream)
     {
         const long long field = (long long)g.nshot * g.plane;
         const float* ez = fused ? pp.Ez[0] : f.Ez;
         const float* hx = fused ? pp.Hx[0] : f.Hx;
         const float* hy = fused ? pp.Hy[0] : f.Hy;
-        launch_tm_pack(P->E[2], (float*)ez, field, true, stream);
-        launch_tm_pack(P->H[0], (float*)hx, field, true, stream);
-        launch_tm_pack(P->H[1], (float*)hy, field, true, stream);
-        if (!fused) return 0;
-        for (int f4 = 0; f4 < 4; ++f4) {
-            if (psi_len_e[f4] && pp.psi_e[0][f4] != home_e[f4] &&
-                hipMemcpyAsync(home_e[f4], pp.psi_e[0][f4], psi_len_e[f4] * 4, hipMemcpyDeviceToDevice, stream) !=
-                    hipSuccess)
-                return -1;
-            if (psi_len_h[f4] && pp.psi_h[0][f4] != home_h[f4] &&
-                hipMemcpyAsync(home_h[f4], pp.psi_h[0][f4], psi_len_h[f4] * 4, hipMemcpyDeviceToDevice, stream) !=
-                    hipSuccess)
-                return -1;
+        TmMoves mv{};
+        mv.add(kTmUnpack, ez, P->E[2], field);
+        mv.add(kTmUnpack, hx, P->H[0], field);
+        mv.add(kTmUnpack, hy, P->H[1], field);
+        for (int f4 = 0; fused && f4 < 4; ++f4) {
+            mv.add(kTmCopy, pp.psi_e[0][f4], home_e[f4], psi_len_e[f4]);
+            mv.add(kTmCopy, pp.psi_h[0][f4], home_h[f4], psi_len_h[f4]);
         }
-        return 0;
+        launch_tm_moves(mv, stream);
     }
 };
 
@@ -1478,10 +1475,7 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
                                     stream));
         }
     }
-    if (tm && tms.unpack(P, stream)) {
-        set_error("forward: copy back of the 2D TM state");
-        return -1;
-    }
+    if (tm) tms.unpack(P, stream);
     if (pl.e_only) {
         if (int8) {
             launch_quant_int8(g, a.Ec, nullptr, 0, int8_writer(pl, P->R_saved, 1, 0), stream);
@@ -1615,15 +1609,13 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
     DevBuf d_goff, d_gshot, d_gcell, d_gmem;
     ReceiverGroups rg{};
     if (adj_rx && !gshot.empty()) {
-        if (!d_goff.alloc(goff.size() * 4) || !d_gshot.alloc(gshot.size() * 4) || !d_gcell.alloc(gcell.size() * 8) ||
-            !d_gmem.alloc(gmem.size() * 4)) {
+        // the fused 2D TM kernels read lists of their own and the members only
+        if (!upload(d_gmem, gmem, stream) ||
+            (!fused && (!upload(d_goff, goff, stream) || !upload(d_gshot, gshot, stream) ||
+                        !upload(d_gcell, gcell, stream)))) {
             set_error("backward: out of device memory for receiver groups");
             return -1;
         }
-        DGX_TRY(hipMemcpyAsync(d_goff.p, goff.data(), goff.size() * 4, hipMemcpyHostToDevice, stream), "upload");
-        DGX_TRY(hipMemcpyAsync(d_gshot.p, gshot.data(), gshot.size() * 4, hipMemcpyHostToDevice, stream), "upload");
-        DGX_TRY(hipMemcpyAsync(d_gcell.p, gcell.data(), gcell.size() * 8, hipMemcpyHostToDevice, stream), "upload");
-        DGX_TRY(hipMemcpyAsync(d_gmem.p, gmem.data(), gmem.size() * 4, hipMemcpyHostToDevice, stream), "upload");
         rg.off = (const int*)d_goff.p;
         rg.shot = (const int*)d_gshot.p;
         rg.cell = (const long long*)d_gcell.p;
@@ -1975,10 +1967,7 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
         launch_copy_spans(back, stream);
     }
     if (xm && nt > 0) TIMED(tmr, kKXmPsiH, launch_xm_psi_h_final(g, kcp, a, stream));
-    if (tm && tms.unpack(P, stream)) {
-        set_error("backward: copy back of the 2D TM state");
-        return -1;
-    }
+    if (tm) tms.unpack(P, stream);
     if (fused && tgrad.terms)  // the last saved step has no later launch to sum it
         TIMED(tmr, kKTmGradReduce,
               launch_tm_grad_reduce(tms.g, pl.box, tgrad.terms, 1, terms_len, mg.want_eps, mg.want_sig, geps, gsig,

@@ -336,7 +336,25 @@ void launch_tm_strip_adj(int order, const Tm2dGrid& g, const Tm2dFields& f, cons
 void launch_tm_fwd_h(int order, const Tm2dGrid& g, const Tm2dFields& f, hipStream_t st);
 void launch_tm_fwd_e(int order, const Tm2dGrid& g, const Tm2dFields& f, const SourceBlocks& src,
                      const HistWrite& hw, hipStream_t st);
-void launch_tm_pack(const float* full, float* compact, long long count, bool unpack, hipStream_t st);
+// Arrays moved in one launch (dgx_tm2d.hip).
+constexpr int kTmMoves = 16;
+enum TmMoveKind : int { kTmCopy = 0, kTmPack, kTmUnpack };
+struct TmMoves {
+    const float* from[kTmMoves];
+    float* to[kTmMoves];
+    long long n[kTmMoves];
+    int kind[kTmMoves];
+    int count;
+    void add(TmMoveKind k, const float* f, float* t, long long len)
+    {
+        if (len <= 0 || f == t) return;
+        from[count] = f;
+        to[count] = t;
+        n[count] = len;
+        kind[count++] = k;
+    }
+};
+void launch_tm_moves(const TmMoves& mv, hipStream_t st);
 void launch_tm_adj_pml(bool electric, const Tm2dGrid& g, const Tm2dFields& f, const Tm2dWeights& w,
                        hipStream_t st);
 void launch_tm_adj_e(int order, const Tm2dGrid& g, const Tm2dFields& f, const Tm2dWeights& w, hipStream_t st);

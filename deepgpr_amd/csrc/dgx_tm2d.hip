@@ -6,6 +6,8 @@
 // expression mirrors the general path (dgx_kernels.hip) with the inactive
 // fields substituted by their exact value 0, including the "+ 0" terms, so
 // both paths agree bit for bit.
+#include <algorithm>
+
 #include "dgx_device.h"
 #include "dgx_internal.h"
 
@@ -195,14 +197,18 @@ __global__ __launch_bounds__(256) void k_tm_fwd_e(Tm2dGrid g, Tm2dFields f, Sour
     if (up || pml || se > sb) f.Ez[n] = ez;
 }
 
-// (nshot, NX, NY, 2) k = 0 plane <-> compact (nshot, NX, NY)
-__global__ __launch_bounds__(256) void k_tm_pack(const float* __restrict__ full, float* __restrict__ compact,
-                                                 long long count, int unpack)
+// The arrays of a solve's compact state in one launch: k = 0 planes of (nshot, NX,
+// NY, 2) arrays to and from compact (nshot, NX, NY) ones, and plain copies. A
+// launch each (and a runtime copy for each CPML auxiliary) was 27 of 3 us a
+// solve.
+__global__ __launch_bounds__(256) void k_tm_move(TmMoves mv)
 {
-    long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= count) return;
-    if (unpack) ((float*)full)[2 * idx] = compact[idx];
-    else compact[idx] = full[2 * idx];
+    const int q = blockIdx.y, kind = mv.kind[q];
+    const float* __restrict__ from = mv.from[q];
+    float* __restrict__ to = mv.to[q];
+    const long long n = mv.n[q];
+    for (long long x = (long long)blockIdx.x * 256 + threadIdx.x; x < n; x += (long long)gridDim.x * 256)
+        to[kind == kTmUnpack ? 2 * x : x] = from[kind == kTmPack ? 2 * x : x];
 }
 
 // --- adjoint ----------------------------------------------------------------
@@ -409,11 +415,13 @@ void launch_tm_fwd_e(int order, const Tm2dGrid& g, const Tm2dFields& f, const So
     else hipLaunchKernelGGL(k_tm_fwd_e<2>, grid, dim3(256), 0, st, g, f, src, hw);
 }
 
-void launch_tm_pack(const float* full, float* compact, long long count, bool unpack, hipStream_t st)
+void launch_tm_moves(const TmMoves& mv, hipStream_t st)
 {
-    if (count <= 0) return;
-    hipLaunchKernelGGL(k_tm_pack, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, full, compact, count,
-                       unpack ? 1 : 0);
+    long long longest = 0;
+    for (int q = 0; q < mv.count; ++q) longest = std::max(longest, mv.n[q]);
+    if (longest <= 0) return;
+    const unsigned blocks = (unsigned)std::min<long long>((longest + 255) / 256, 1024);
+    hipLaunchKernelGGL(k_tm_move, dim3(blocks, (unsigned)mv.count), dim3(256), 0, st, mv);
 }
 
 void launch_tm_adj_pml(bool electric, const Tm2dGrid& g, const Tm2dFields& f, const Tm2dWeights& w,
