@@ -2725,6 +2725,25 @@ DGX_API void dgx_batch_destroy(void* batch)
     delete b;  // the retired memory too: every event has completed
 }
 
+DGX_API int dgx_model_checks(const float* er, const float* se, const float* mr, long long cells, const float* wave,
+                             long long nwave, const void* src, int src_bytes, long long nsrc, const void* rx,
+                             int rx_bytes, long long nrx, int nx, int ny, int nz, float* out, int blocks,
+                             dgx_stream_t stream)
+{
+    g_error[0] = '\0';
+    if (!er || !se || !mr || !wave || !src || !rx || !out || cells <= 0 || nwave < 0 || nsrc < 0 || nrx < 0 ||
+        nsrc % 3 || nrx % 3 || (src_bytes != 4 && src_bytes != 8) || (rx_bytes != 4 && rx_bytes != 8) ||
+        blocks <= 0 || blocks > 65535) {
+        set_error("model checks: invalid argument");
+        return -1;
+    }
+    const ModelChecks m{er, se, mr, wave, src, rx, cells, nwave, nsrc, nrx, src_bytes == 8, rx_bytes == 8,
+                        {nx, ny, nz}, out};
+    launch_model_checks(m, blocks, (hipStream_t)stream);
+    DGX_TRY(hipGetLastError(), "model checks: kernel launch");
+    return 0;
+}
+
 DGX_API int dgx_codec_roundtrip(const float* input, void* encoded, float* decoded, long long count,
                                 int storage_kind, int conversion_backend, dgx_stream_t stream)
 {

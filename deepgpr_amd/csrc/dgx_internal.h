@@ -336,6 +336,19 @@ void launch_tm_strip_adj(int order, const Tm2dGrid& g, const Tm2dFields& f, cons
 void launch_tm_fwd_h(int order, const Tm2dGrid& g, const Tm2dFields& f, hipStream_t st);
 void launch_tm_fwd_e(int order, const Tm2dGrid& g, const Tm2dFields& f, const SourceBlocks& src,
                      const HistWrite& hw, hipStream_t st);
+// Value checks of a solve's inputs (dgx_checks.hip): material arrays of `cells`
+// cells, waveform samples, coordinates (3 a location, 32 or 64 bits).
+constexpr int kModelChecks = 11;
+struct ModelChecks {
+    const float *er, *se, *mr, *wave;
+    const void *src, *rx;
+    long long cells, nwave, nsrc, nrx;  // nsrc, nrx: coordinates
+    int src64, rx64;
+    int shape[3];
+    float* out;  // blocks x kModelChecks
+};
+void launch_model_checks(const ModelChecks& m, int blocks, hipStream_t st);
+
 // Arrays moved in one launch (dgx_tm2d.hip).
 constexpr int kTmMoves = 16;
 enum TmMoveKind : int { kTmCopy = 0, kTmPack, kTmUnpack };

@@ -126,6 +126,11 @@ NATIVE_FUNCTIONS: Dict[str, Tuple[tuple, object]] = {
     "dgx_forward_noalloc_scratch_bytes": ((), LONGLONG),
     "dgx_tm2d_tile_rows_tuned": ((("nx_fields", INT), ("ny_fields", INT), ("nshot", INT), ("order", INT),
                                   ("cpml", INT)), INT),
+    "dgx_model_checks": ((("er", VOID_PTR), ("se", VOID_PTR), ("mr", VOID_PTR), ("cells", LONGLONG),
+                          ("wave", VOID_PTR), ("nwave", LONGLONG), ("src", VOID_PTR), ("src_bytes", INT),
+                          ("nsrc", LONGLONG), ("rx", VOID_PTR), ("rx_bytes", INT), ("nrx", LONGLONG),
+                          ("nx", INT), ("ny", INT), ("nz", INT), ("out", VOID_PTR), ("blocks", INT),
+                          ("stream", VOID_PTR)), INT),
     "dgx_codec_roundtrip": ((("input", FLOAT_PTR), ("encoded", VOID_PTR), ("decoded", FLOAT_PTR),
                              ("count", LONGLONG), ("storage_kind", INT),
                              ("conversion_backend", INT), ("stream", VOID_PTR)), INT),

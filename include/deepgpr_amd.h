@@ -132,6 +132,17 @@ DGX_API long long dgx_forward_noalloc_scratch_bytes(void);
  * several steps a launch (orders 2 and 4) has no use for it and is not timed:
  * it reports the height that the rule by size gives. */
 DGX_API int dgx_tm2d_tile_rows_tuned(int nx_fields, int ny_fields, int nshot, int order, int cpml);
+/* No counterpart in the reference. The value checks of a solve's inputs in one
+ * pass over device arrays: er, se and mr of `cells` cells, nwave waveform
+ * samples, nsrc and nrx int32 or int64 coordinates (src_bytes, rx_bytes: 4 or
+ * 8), three a location. Each of the `blocks` workgroups writes 11 floats to
+ * out, to be combined by their minimum: 1 or 0 for finite er, se, mr and wave;
+ * the least er, se, mr, er * mr and -se; 1 or 0 for sources and receivers in
+ * [0, n) of an nx x ny x nz grid. */
+DGX_API int dgx_model_checks(const float* er, const float* se, const float* mr, long long cells, const float* wave,
+                             long long nwave, const void* src, int src_bytes, long long nsrc, const void* rx,
+                             int rx_bytes, long long nrx, int nx, int ny, int nz, float* out, int blocks,
+                             dgx_stream_t stream);
 /* FP16/BF16 history codec round trip on device arrays; replaces
  * deepgpr_test_wavefield_conversion (deepgpr.h:84-86). */
 DGX_API int dgx_codec_roundtrip(const float* input, void* encoded, float* decoded, long long count,
