@@ -598,8 +598,9 @@ __device__ __forceinline__ void fwd_e_group(const Grid& g, const float* ca, cons
     }
     const fv<V> hx = ldv<V>(Hf.c[0], q.m), hy = ldv<V>(Hf.c[1], q.m);
     fv<V> e[3] = {ldv<V>(E.c[0], q.m), ldv<V>(E.c[1], q.m), ldv<V>(E.c[2], q.m)};
-    const fv<V> eold[3] = {e[0], e[1], e[2]};
-    const fv<V> u0 = ldv<V>(ca, q.m), u1 = ldv<V>(ccurl, q.m), cbv = ldv<V>(cb, q.m);
+    const fv<V> u0 = ldv<V>(ca, q.m), u1 = ldv<V>(ccurl, q.m);
+    fv<V> cbv = 0.0f;
+    if constexpr (!XY) cbv = ldv<V>(cb, q.m);
     const bool lx = q.i >= 1, ly = q.j >= 1;
     stv<V>(s0, (unsigned)q.k, hx, q.dup);
     stv<V>(s1, (unsigned)q.k, hy, q.dup);
@@ -625,10 +626,15 @@ __device__ __forceinline__ void fwd_e_group(const Grid& g, const float* ca, cons
         const ZFace<V> zf = z_face<V, true>(g, cp, tab, cb, q);
         if (zf.any) z_face_apply<V, true>(g, q, zf, dyz, dxz, e[0], e[1]);
     }
+    // sources and the history load cb, and the history ca and the old values,
+    // again rather than keep them in registers all along
+    unsigned m = q.m;
+    asm volatile("" : "+v"(m));
     for (int x = sb; x < se; ++x) {
         const int2 ent = src.entries[x];
         const unsigned at = (unsigned)ent.x - q.m;
         if (at < (unsigned)V) {
+            const fv<V> cbv = ldv<V>(cb, m);
             const float scale = src.wave[(long long)ent.y * src.nt + src.it] * src.dl / src.vol;
 #pragma unroll
             for (int y = 0; y < V; ++y)
@@ -646,19 +652,25 @@ __device__ __forceinline__ void fwd_e_group(const Grid& g, const float* ca, cons
         bool own[V];
 #pragma unroll
         for (int y = 0; y < V; ++y) own[y] = y >= q.dup && z + y >= 0 && z + y < hist.box.nz;
+        fv<V> cbv = 0.0f, cav = 0.0f;
+        if (hist.save_r) {
+            cbv = ldv<V>(cb, m);
+            cav = ldv<V>(ca, m);
+        }
 #pragma unroll
         for (int comp = 0; comp < 3; ++comp) {
             if (hist.mode != 3 && comp != 2) continue;
             const int ci = hist.mode == 3 ? comp : 0;
+            const fv<V> old = ldv<V>(E.c[comp], m);
             if (hist.save_e)
-                store_hist_group<V>(hist.e_base, ci * hist.e_cstride + base, eold[comp], hist.e_kind, whole, own);
+                store_hist_group<V>(hist.e_base, ci * hist.e_cstride + base, old, hist.e_kind, whole, own);
             if (hist.save_r) {
                 fv<V> rhs;
 #pragma unroll
                 for (int y = 0; y < V; ++y) {
                     const bool u = up[comp] && q.k + y < n2 - 1 && (comp == 2 || q.k + y > 0);
-                    const float a = u ? u0[y] : 1.0f;
-                    rhs[y] = cbv[y] != 0.0f ? (e[comp][y] - a * eold[comp][y]) / cbv[y] : 0.0f;
+                    const float a = u ? cav[y] : 1.0f;
+                    rhs[y] = cbv[y] != 0.0f ? (e[comp][y] - a * old[y]) / cbv[y] : 0.0f;
                 }
                 store_hist_group<V>(hist.r_base, ci * hist.r_cstride + base, rhs, hist.r_kind, whole, own);
             }
@@ -984,9 +996,6 @@ __device__ __forceinline__ void adj_group(const Grid& g, const float* cu, const 
     const int sx = g.plane, sy = g.N[2], n2 = g.N[2];
     const fv<V> l[3] = {ldv<V>(lam.c[0], q.m), ldv<V>(lam.c[1], q.m), ldv<V>(lam.c[2], q.m)};
     const fv<V> ku = ldv<V>(cu, q.m);
-    fv<V> o[3] = {ldv<V>(out.c[0], q.m), ldv<V>(out.c[1], q.m), ldv<V>(out.c[2], q.m)};
-    fv<V> cav = 0.0f;
-    if (!EL) cav = ldv<V>(ca, q.m);
     // the z-channel weights of the own cells, shared with the row
     fv<V> w0 = 0.0f, w1 = 0.0f;
     if (!q.zplain && has_cpml) {
@@ -1029,6 +1038,12 @@ __device__ __forceinline__ void adj_group(const Grid& g, const float* cu, const 
         y0 = pick_z<V, !EL>(io, q.k, n2, y0, none);
         y2 = pick_z<V, EL>(ii, q.k, n2, y2, none);
     }
+    // loaded here, not before the gathers: 16 registers less all along
+    unsigned m = q.m;
+    asm volatile("" : "+v"(m));
+    fv<V> o[3] = {ldv<V>(out.c[0], m), ldv<V>(out.c[1], m), ldv<V>(out.c[2], m)};
+    fv<V> cav = 0.0f;
+    if (!EL) cav = ldv<V>(ca, m);
     __syncthreads();
     gather_z<ORDER, V, EL>(q, n2, s0, s1, w0, w1, z0, z1);
     if (!EL) {
