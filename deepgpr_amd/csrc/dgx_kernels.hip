@@ -9,6 +9,8 @@
 #include <cstdlib>
 #include <cstring>
 
+#include <type_traits>
+
 #include "dgx_device.h"
 #include "dgx_internal.h"
 
@@ -547,7 +549,10 @@ __global__ __launch_bounds__(64) void k_adj_source(Grid g, const int* __restrict
 // ---------------------------------------------------------------------------
 // Material gradient fused with the history decode (deepgpr_cpu.c:1659-1745)
 // ---------------------------------------------------------------------------
-template <typename ACC>
+// KIND and the number of components are constants, so that all of a shot's loads
+// (9 for three components) and the sums are in flight before the first use; with
+// a loop over the components a cell waited for memory once a component.
+template <typename ACC, int KIND, int COMPS>
 __global__ __launch_bounds__(256) void k_material_gradient(Grid g, CF3 L, MatGrad mg, ACC* __restrict__ geps,
                                                            ACC* __restrict__ gsig)
 {
@@ -572,12 +577,12 @@ __global__ __launch_bounds__(256) void k_material_gradient(Grid g, CF3 L, MatGra
     const long long m = (long long)ix * g.st0 + (long long)iy * g.N[2] + iz;
     const long long out = ((long long)ix * (g.N[1] - 1) + iy) * (g.N[2] - 1) + iz;
     const float cav = mg.ca[m], cbv = mg.cb[m];
-    const bool active = mg.sig[m] <= kPecSigma;
-    const int comps = mg.mode == 3 ? 3 : 1;
+    const float sig = mg.sig[m];
+    const ACC ge0 = mg.want_eps ? geps[out] : (ACC)0, gs0 = mg.want_sig ? gsig[out] : (ACC)0;
     const float wgt = (float)mg.weight;
     // the INT8 tiles of this cell, formed once for every shot and component
     long long tile_e = 0, tile_s = 0;
-    if (mg.kind == kInt8) {
+    if constexpr (KIND == kInt8) {
         tile_e = int8_tile(mg.e8, ix - b.x0, iy - b.y0, iz - b.z0);
         tile_s = int8_tile(mg.s8, ix - b.x0, iy - b.y0, iz - b.z0);
     }
@@ -585,42 +590,40 @@ __global__ __launch_bounds__(256) void k_material_gradient(Grid g, CF3 L, MatGra
     for (int s = 0; s < g.nshot; ++s) {
         const long long f = (long long)s * g.cells + m;
         const long long base = (long long)s * b.cells + h;
-        for (int ci = 0; ci < comps; ++ci) {
-            const int comp = mg.mode == 3 ? ci : 2;
-            const bool up = e_updated(g, comp, c);
-            float e_old, sec;
-            if (mg.kind == kInt8) {
-                e_old = int8_load_at(mg.e8, b, ci, s, h, tile_e);
-                sec = int8_load_at(mg.s8, b, ci, s, h, tile_s);
+        float e_old[COMPS], sec[COMPS], lam[COMPS];
+#pragma unroll
+        for (int ci = 0; ci < COMPS; ++ci) {
+            if constexpr (KIND == kInt8) {
+                e_old[ci] = int8_load_at(mg.e8, b, ci, s, h, tile_e);
+                sec[ci] = int8_load_at(mg.s8, b, ci, s, h, tile_s);
             } else {
-                e_old = load_hist(mg.eframe, ci * mg.e_cstride + base, mg.kind);
-                sec = load_hist(mg.sframe, ci * mg.s_cstride + base, mg.kind);
+                e_old[ci] = load_hist(mg.eframe, ci * mg.e_cstride + base, KIND);
+                sec[ci] = load_hist(mg.sframe, ci * mg.s_cstride + base, KIND);
             }
-            float lam = L.c[comp][f];
-            float rhs = sec;
+            lam[ci] = L.c[COMPS == 3 ? ci : 2][f];
+        }
+        const bool active = sig <= kPecSigma;
+        const float eca = kEps0 * (1.0f - cav) * cbv / mg.dt, ecb = -kEps0 * cbv * cbv / mg.dt;
+        const float sca = -0.5f * (1.0f + cav) * cbv, scb = -0.5f * cbv * cbv;
+#pragma unroll
+        for (int ci = 0; ci < COMPS; ++ci) {
+            const bool up = e_updated(g, COMPS == 3 ? ci : 2, c);
+            float l = lam[ci], rhs = sec[ci];
             if (mg.e_only) {
                 const float a = up ? cav : 1.0f;
-                rhs = cbv != 0.0f ? (sec - a * e_old) / cbv : 0.0f;
+                rhs = cbv != 0.0f ? (sec[ci] - a * e_old[ci]) / cbv : 0.0f;
             }
-            if (e_old == 0.0f && rhs == 0.0f) lam = 0.0f;
-            const float gca = up ? lam * e_old * wgt : 0.0f;
-            const float gcb = lam * rhs * wgt;
+            if (e_old[ci] == 0.0f && rhs == 0.0f) l = 0.0f;
+            const float gca = up ? l * e_old[ci] * wgt : 0.0f;
+            const float gcb = l * rhs * wgt;
             if (active) {
-                if (mg.want_eps) {
-                    const float dca = kEps0 * (1.0f - cav) * cbv / mg.dt;
-                    const float dcb = -kEps0 * cbv * cbv / mg.dt;
-                    ge += (ACC)(gca * dca + gcb * dcb);
-                }
-                if (mg.want_sig) {
-                    const float dca = -0.5f * (1.0f + cav) * cbv;
-                    const float dcb = -0.5f * cbv * cbv;
-                    gs += (ACC)(gca * dca + gcb * dcb);
-                }
+                if (mg.want_eps) ge += (ACC)(gca * eca + gcb * ecb);
+                if (mg.want_sig) gs += (ACC)(gca * sca + gcb * scb);
             }
         }
     }
-    if (mg.want_eps) geps[out] += ge;
-    if (mg.want_sig) gsig[out] += gs;
+    if (mg.want_eps) geps[out] = ge0 + ge;
+    if (mg.want_sig) gsig[out] = gs0 + gs;
 }
 
 __global__ __launch_bounds__(256) void k_add_f64_to_f32(const double* __restrict__ a, float* __restrict__ out,
@@ -1028,13 +1031,24 @@ void launch_adj_source(const Grid& g, const int* loc, const float* cb, const flo
 void launch_material_gradient(const Grid& g, CF3 L, const MatGrad& mg, void* geps, void* gsig, bool fp64,
                               hipStream_t st)
 {
-    unsigned blocks = (unsigned)((mg.box.cells + 255) / 256);
-    if (fp64)
-        hipLaunchKernelGGL(k_material_gradient<double>, dim3(blocks), dim3(256), 0, st, g, L, mg, (double*)geps,
-                           (double*)gsig);
-    else
-        hipLaunchKernelGGL(k_material_gradient<float>, dim3(blocks), dim3(256), 0, st, g, L, mg, (float*)geps,
-                           (float*)gsig);
+    const dim3 blocks((unsigned)((mg.box.cells + 255) / 256));
+    auto go = [&](auto acc, auto kind, auto comps) {
+        typedef decltype(acc) ACC;
+        hipLaunchKernelGGL((k_material_gradient<ACC, decltype(kind)::value, decltype(comps)::value>), blocks, dim3(256),
+                           0, st, g, L, mg, (ACC*)geps, (ACC*)gsig);
+    };
+    auto of_kind = [&](auto acc, auto comps) {
+        if (mg.kind == kInt8) go(acc, std::integral_constant<int, kInt8>(), comps);
+        else if (mg.kind == kF16) go(acc, std::integral_constant<int, kF16>(), comps);
+        else if (mg.kind == kBF16) go(acc, std::integral_constant<int, kBF16>(), comps);
+        else go(acc, std::integral_constant<int, kF32>(), comps);
+    };
+    auto of_comps = [&](auto acc) {
+        if (mg.mode == 3) of_kind(acc, std::integral_constant<int, 3>());
+        else of_kind(acc, std::integral_constant<int, 1>());
+    };
+    if (fp64) of_comps(0.0);
+    else of_comps(0.0f);
 }
 
 void launch_add_f64(const double* a, float* out, long long count, hipStream_t st)

@@ -16,10 +16,14 @@
 // fewer cells a thread were slower (two cells: 2 % on 289 x 289 x 225 fields,
 // 17 % on 161 x 161 x 129 x 4 shots). Measured on an MI355X, order 4, CPML 16,
 // 289 x 289 x 225 fields, us per launch, before (one thread per cell, stored
-// weights) and now: forward H 283 and 251, forward E 286 and 293, adjoint 1038
-// (three launches) and 676 (two). What bounds them now is the chain of a
-// wavefront (loads, row exchange, z-CPML loads, stores) at 3 to 4 wavefronts a
-// SIMD, not the bytes.
+// weights) and now: forward H 283 and 250, forward E 286 and 263, adjoint 1038
+// (three launches) and 629 (two). What bounds them now is the chain of a
+// wavefront (loads, row exchange, z-CPML loads, stores) at 4 wavefronts a SIMD,
+// not the bytes. Four need at most 128 registers a lane, so what only the end of
+// a sweep uses is loaded there: with the old fields, cb and the adjoint's outputs
+// held from the start (136 to 140 registers, 3 wavefronts) forward E took 293 and
+// the adjoint 677. At 96 registers (5 wavefronts) the plain groups spill: forward
+// 396 and 570, adjoint 1052.
 #include <algorithm>
 
 #include "dgx_device.h"
