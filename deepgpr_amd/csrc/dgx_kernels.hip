@@ -512,6 +512,82 @@ __global__ __launch_bounds__(256) void k_quant_int8_w64(Grid g, CF3 E, const flo
     }
 }
 
+// The same for 4x4x4 tiles, the default of 3D histories: four tiles that follow
+// one another along z per wavefront, four z cells a lane. One cell a lane makes a
+// load of 16 pieces of 16 bytes and a store of 16 pieces of 4; here they are 64
+// and 16 bytes. 161 x 161 x 129, four shots, three components: 160 us with one
+// tile a wavefront, 55 now. Lane 4 r + t holds row r = 4 lx + ly of tile t; the
+// maximum pairs the 64 cells (index 4 r + lz) as above: rows 8, 4, 2 and 1 apart
+// through shuffles, then lz 2 and 1 apart.
+__global__ __launch_bounds__(256) void k_quant_int8_444(Grid g, CF3 E, const float* __restrict__ src,
+                                                        long long src_cstride, Int8Write w, int groups, int nzg,
+                                                        Div div_nzg, Div div_plane)
+{
+    const int lane = threadIdx.x & 63;
+    const int group = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    if (group >= groups) return;  // whole wavefronts
+    const int s = blockIdx.y, ci = blockIdx.z, comp = w.mode == 3 ? ci : 2;
+    const unsigned trow = div_q((unsigned)group, div_nzg), tx = div_q((unsigned)group, div_plane);
+    const int ty = (int)(trow - tx * (unsigned)w.nby), tz = (group - (int)(trow * (unsigned)nzg)) * 4 + (lane & 3);
+    const int row = lane >> 2;
+    const int x = (int)tx * 4 + (row >> 2), y = ty * 4 + (row & 3), z = tz * 4;
+    const int n = x < w.box.nx && y < w.box.ny ? min(max(w.box.nz - z, 0), 4) : 0;  // cells of the lane
+    const long long h = n > 0 ? ((long long)x * w.box.ny + y) * w.box.nz + z : 0;
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef signed char c4 __attribute__((ext_vector_type(4), aligned(1)));
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (n > 0) {
+        const float* p = src ? src + ci * src_cstride + (long long)s * w.box.cells + h
+                             : E.c[comp] + (long long)s * g.cells + (long long)(x + w.box.x0) * g.st0 +
+                                   (long long)(y + w.box.y0) * g.N[2] + (z + w.box.z0);
+        if (n == 4) {
+            const f4 a = *(const f4*)p;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = a[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (e < n) v[e] = p[e];
+        }
+    }
+    float m[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m[e] = v[e] < 0.0f ? -v[e] : v[e];
+#pragma unroll
+    for (int stride = 32; stride >= 4; stride >>= 1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float o = __shfl_down(m[e], stride, 64);
+            if (o > m[e]) m[e] = o;  // lanes of the upper half keep values that are not used again
+        }
+    }
+    if (m[2] > m[0]) m[0] = m[2];
+    if (m[3] > m[1]) m[1] = m[3];
+    if (m[1] > m[0]) m[0] = m[1];
+    const float peak = __shfl(m[0], lane & 3, 64);
+    const float scale = peak >= 1.0e-30f ? peak / 127.0f : 1.0f;
+    const int tile = (int)trow * w.nbz + tz;
+    if (row == 0 && tz < w.nbz)
+        w.scale[((long long)ci * w.frames + w.frame) * g.nshot * w.tiles + (long long)s * w.tiles + tile] = scale;
+    if (n > 0) {
+        signed char* q = w.q + ((long long)ci * w.frames + w.frame) * ((long long)g.nshot * w.box.cells) +
+                         (long long)s * w.box.cells + h;
+        c4 b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float r = fminf(fmaxf(rintf(v[e] / scale), -127.0f), 127.0f);
+            b[e] = (signed char)(int)r;
+        }
+        if (n == 4) {
+            *(c4*)q = b;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (e < n) q[e] = b[e];
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Adjoint: receivers^T and source^T (deepgpr_cpu.c:1479-1534)
 // ---------------------------------------------------------------------------
@@ -1004,6 +1080,13 @@ void launch_quant_int8(const Grid& g, CF3 E, const float* src, long long src_cst
                        hipStream_t st)
 {
     int comps = w.mode == 3 ? 3 : 1;
+    if (w.bx == 4 && w.by == 4 && w.bz == 4) {
+        const int nzg = (w.nbz + 3) / 4, groups = (int)(w.tiles / w.nbz) * nzg;
+        const dim3 grid((unsigned)((groups + 3) / 4), (unsigned)g.nshot, (unsigned)comps);
+        hipLaunchKernelGGL(k_quant_int8_444, grid, dim3(256), 0, st, g, E, src, src_cstride, w, groups, nzg,
+                           make_div((unsigned)nzg), make_div((unsigned)(nzg * w.nby)));
+        return;
+    }
     if (w.bx * w.by * w.bz == 64) {
         dim3 grid((unsigned)((w.tiles + 3) / 4), (unsigned)g.nshot, (unsigned)comps);
         hipLaunchKernelGGL(k_quant_int8_w64, grid, dim3(256), 0, st, g, E, src, src_cstride, w);
