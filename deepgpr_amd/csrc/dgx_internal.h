@@ -368,6 +368,7 @@ struct TmMoves {
     }
 };
 void launch_tm_moves(const TmMoves& mv, hipStream_t st);
+void launch_tm_zero(void* p, long long bytes, hipStream_t st);  // whole 2-byte elements
 void launch_tm_adj_pml(bool electric, const Tm2dGrid& g, const Tm2dFields& f, const Tm2dWeights& w,
                        hipStream_t st);
 void launch_tm_adj_e(int order, const Tm2dGrid& g, const Tm2dFields& f, const Tm2dWeights& w, hipStream_t st);

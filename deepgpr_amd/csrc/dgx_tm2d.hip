@@ -211,6 +211,19 @@ __global__ __launch_bounds__(256) void k_tm_move(TmMoves mv)
         to[kind == kTmUnpack ? 2 * x : x] = from[kind == kTmPack ? 2 * x : x];
 }
 
+// Zeroes bytes of an array of 2- or 4-byte elements, 16 a lane.
+__global__ __launch_bounds__(256) void k_tm_zero(char* __restrict__ p, long long bytes)
+{
+    typedef unsigned v4 __attribute__((ext_vector_type(4)));
+    const long long head = min((long long)((16 - (long long)((unsigned long long)p & 15)) & 15), bytes);
+    const long long vecs = (bytes - head) / 16, first = (long long)blockIdx.x * 256 + threadIdx.x;
+    for (long long x = first; x < vecs; x += (long long)gridDim.x * 256)
+        __builtin_nontemporal_store((v4)(0u), (v4*)(p + head) + x);
+    const long long tail = head + vecs * 16;
+    if (2 * first < head) *(unsigned short*)(p + 2 * first) = 0;
+    if (tail + 2 * first < bytes) *(unsigned short*)(p + tail + 2 * first) = 0;
+}
+
 // --- adjoint ----------------------------------------------------------------
 
 template <bool ELECTRIC>
@@ -413,6 +426,13 @@ void launch_tm_fwd_e(int order, const Tm2dGrid& g, const Tm2dFields& f, const So
     if (order == 8) hipLaunchKernelGGL(k_tm_fwd_e<8>, grid, dim3(256), 0, st, g, f, src, hw);
     else if (order == 4) hipLaunchKernelGGL(k_tm_fwd_e<4>, grid, dim3(256), 0, st, g, f, src, hw);
     else hipLaunchKernelGGL(k_tm_fwd_e<2>, grid, dim3(256), 0, st, g, f, src, hw);
+}
+
+void launch_tm_zero(void* p, long long bytes, hipStream_t st)
+{
+    if (bytes <= 0) return;
+    const unsigned blocks = (unsigned)std::min<long long>((bytes + 4095) / 4096, 8192);
+    hipLaunchKernelGGL(k_tm_zero, dim3(blocks), dim3(256), 0, st, (char*)p, bytes);
 }
 
 void launch_tm_moves(const TmMoves& mv, hipStream_t st)

@@ -27,13 +27,16 @@ CASES = [
     (100, 105, 2, 11, 17, 2, "bf16", 3, (6, 0, 5, 7), (0.018, 0.02), True),
     (61, 209, 4, 5, 26, 1, "bf16", 2, (6, 9, 10, 5), (0.02, 0.02), False),
     (64, 105, 2, 8, 43, 2, "f32", 3, (6, 9, 10, 5), (0.02, 0.019), True),
+    (52, 62, 2, 9, 1, 1, "e_only", 3, (7, 6, 5, 8), (0.02, 0.02), False),
+    (46, 38, 4, 7, 3, 2, "f16_e", 3, (6, 5, 7, 3), (0.02, 0.018), True),
     (300, 700, 2, 9, 1, 2, "f32", 3, (10, 7, 9, 10), (0.02, 0.02), True),
     (251, 731, 4, 5, 1, 1, "e_only", 2, (10, 7, 9, 10), (0.02, 0.021), False),
 ]
 
 
 def _storage(h, name):
-    return {"f32": 0, "e_only": h.RHS_FROM_E, "f16": h.KIND_F16, "bf16": h.KIND_BF16}[name]
+    return {"f32": 0, "e_only": h.RHS_FROM_E, "f16": h.KIND_F16, "bf16": h.KIND_BF16,
+            "f16_e": h.KIND_F16 | h.RHS_FROM_E}[name]
 
 
 def _problem(h, case):
