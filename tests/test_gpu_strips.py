@@ -28,7 +28,7 @@ CASES = [
     (61, 209, 4, 5, 26, 1, "bf16", 2, (6, 9, 10, 5), (0.02, 0.02), False),
     (64, 105, 2, 8, 43, 2, "f32", 3, (6, 9, 10, 5), (0.02, 0.019), True),
     (52, 62, 2, 9, 1, 1, "e_only", 3, (7, 6, 5, 8), (0.02, 0.02), False),
-    (46, 38, 4, 7, 3, 2, "f16_e", 3, (6, 5, 7, 3), (0.02, 0.018), True),
+    (46, 38, 4, 7, 3, 1, "f16_e", 3, (6, 5, 7, 3), (0.02, 0.018), True),
     (300, 700, 2, 9, 1, 2, "f32", 3, (10, 7, 9, 10), (0.02, 0.02), True),
     (251, 731, 4, 5, 1, 1, "e_only", 2, (10, 7, 9, 10), (0.02, 0.021), False),
 ]
