@@ -7,7 +7,9 @@
 // row: its first cells belong to the group before it. There are two kinds of
 // workgroups: plain ones, whose rows lie in the plain ranges of x and y, with
 // groups of V cells, and edge ones with groups of V / 2 cells (their code holds
-// more values a cell).
+// more values a cell). The first threads of a workgroup take the groups at the
+// ends of its rows, so that one or two wavefronts run the z-CPML and the z-edge
+// code and the others skip it.
 #pragma once
 
 #include "dgx_sweep.h"
@@ -17,7 +19,9 @@ namespace dgx {
 struct RowKind {
     int gpr;   // groups of a row
     int rb;    // rows of a workgroup
-    Div div;   // / gpr
+    int ends;  // groups of a row that reach out of the plain z-range
+    int low;   // of these, the ones at its start
+    Div div_ends, div_mid;  // / ends, / (gpr - ends), or / 1
 };
 
 struct RowMap {
@@ -75,7 +79,6 @@ inline RowKind make_row_kind(int n2, int V, int max_threads)
 {
     RowKind k{};
     k.gpr = (n2 + V - 1) / V;
-    k.div = make_div((unsigned)k.gpr);
     double best = 0.0;
     for (int rb = 1; rb <= 16; ++rb) {
         const int t = (rb * k.gpr + 63) / 64 * 64;
@@ -87,6 +90,18 @@ inline RowKind make_row_kind(int n2, int V, int max_threads)
         }
     }
     return k;
+}
+
+// Groups at the ends of a row: not wholly in the plain z-range.
+inline void set_row_ends(RowKind& k, int V, int zlo, int zhi)
+{
+    const int low = (zlo + V - 1) / V, from = (zhi + 1) / V;  // groups below zlo; the first group beyond zhi
+    k.low = low < k.gpr ? low : k.gpr;
+    const int high = k.gpr - (from > k.low ? from : k.low);
+    k.ends = k.low + (high > 0 ? high : 0);
+    if (k.ends >= k.gpr) k.ends = k.low = 0;  // no others
+    k.div_ends = make_div((unsigned)(k.ends > 0 ? k.ends : 1));
+    k.div_mid = make_div((unsigned)(k.gpr > k.ends ? k.gpr - k.ends : 1));
 }
 
 inline RowMap make_row_map(const int N[3], const int pml[6], int R, int V, int max_threads)
@@ -101,6 +116,8 @@ inline RowMap make_row_map(const int N[3], const int pml[6], int R, int V, int m
     row_plain_range(N[2], pml[4], pml[5], R, m.zlo, m.zhi);
     m.plain = make_row_kind(N[2], V, max_threads);
     m.edge = make_row_kind(N[2], V / 2, max_threads);
+    set_row_ends(m.plain, V, m.zlo, m.zhi);
+    set_row_ends(m.edge, V / 2, m.zlo, m.zhi);
     const int tp = m.plain.rb * m.plain.gpr, te = m.edge.rb * m.edge.gpr;
     m.threads = ((tp > te ? tp : te) + 63) / 64 * 64;
     const int lp = tp * V, le = te * (V / 2);
@@ -159,13 +176,23 @@ DGX_HD int row_block(const RowMap& m, int b, int& i, int& j0, int& nj)
     return nj > 0 ? 1 : -1;
 }
 
-// Thread t of a workgroup of nj rows: its row, the first cell k of its group of
+// Thread t of a workgroup of nj rows (the ends of its rows first, then what lies
+// between them, row by row): its row, the first cell k of its group of
 // V cells and how many of the group's first cells belong to the group before
 // it; false for an idle thread (row, k and dup are then those of a valid one).
 DGX_HD bool row_thread(const RowMap& m, const RowKind& kd, int V, int t, int nj, int& row, int& k, int& dup)
 {
-    row = (int)div_q((unsigned)t, kd.div);
-    k = (t - row * kd.gpr) * V;
+    const int u = t - kd.rb * kd.ends;
+    if (u < 0) {
+        row = (int)div_q((unsigned)t, kd.div_ends);
+        k = t - row * kd.ends;
+        if (k >= kd.low) k += kd.gpr - kd.ends;
+    } else {
+        const int mid = kd.gpr - kd.ends;
+        row = (int)div_q((unsigned)u, kd.div_mid);
+        k = u - row * mid + kd.low;
+    }
+    k *= V;
     dup = 0;
     if (k > m.n2 - V) {
         dup = k - (m.n2 - V);

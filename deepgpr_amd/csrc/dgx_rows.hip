@@ -5,22 +5,27 @@
 // 40 B a cell, plus 8 B an active CPML auxiliary. The adjoint therefore forms
 // the weights of its transposed stencils where it reads them (one product, or
 // in the CPML the auxiliary's term) instead of storing six arrays of them
-// between two sweeps. A thread's taps along x and y are one V-wide load each.
-// A workgroup covers whole rows, the z-CPML included, so every cache line is
-// fetched and written once; the few lanes at the ends of a row do the z-CPML
-// work beside the others. Rows away from the x and y faces (the whole
-// workgroup) run code without any test of those axes (XY).
+// between two sweeps. A thread's taps along x and y are one V-wide load each. A
+// workgroup covers whole rows, the z-CPML included, so every cache line is
+// fetched and written once; the ends of its rows, with the z-CPML work, are put
+// into as few of its wavefronts as hold them. Rows away from the x and y faces
+// (the whole workgroup) run code without any test of those axes (XY).
 //
 // Four cells a thread in plain rows: a 64-lane load then moves 1 KiB, where a
 // load of one float a lane occupies the address unit nearly as long; wider or
 // fewer cells a thread were slower (two cells: 2 % on 289 x 289 x 225 fields,
 // 17 % on 161 x 161 x 129 x 4 shots). Measured on an MI355X, order 4, CPML 16,
 // 289 x 289 x 225 fields, us per launch, before (one thread per cell, stored
-// weights) and now: forward H 283 and 250, forward E 286 and 263, adjoint 1038
-// (three launches) and 629 (two). What bounds them now is the chain of a
-// wavefront (loads, row exchange, z-CPML loads, stores) at 4 wavefronts a SIMD,
-// not the bytes. Four need at most 128 registers a lane, so what only the end of
-// a sweep uses is loaded there: with the old fields, cb and the adjoint's outputs
+// weights) and now: forward H 283 and 229, forward E 286 and 248, adjoint 1038
+// (three launches) and 615 (two). With the ends of the rows in every wavefront
+// these were 243, 256 and 607; 129 x 129 x 129 x 2 shots, order 4, 63, 73 and 189
+// against 58, 68 and 179 now; order 2 on 165 x 141 x 189, 45, 51 and 101 against
+// 42, 45 and 98. What bounds them now is the chain of a wavefront (loads, row
+// exchange, z-CPML loads, stores) at 4 wavefronts a SIMD and, in the adjoint,
+// the vector instructions (62 % of the cycles), not the bytes.
+//
+// Four wavefronts need at most 128 registers a lane, so what only the end of a
+// sweep uses is loaded there: with the old fields, cb and the adjoint's outputs
 // held from the start (136 to 140 registers, 3 wavefronts) forward E took 293 and
 // the adjoint 677. At 96 registers (5 wavefronts) the plain groups spill: forward
 // 396 and 570, adjoint 1052.
@@ -486,9 +491,16 @@ __device__ __forceinline__ void fwd_h_group(const Grid& g, const float* hcurl, c
     __syncthreads();
     const fv<V> dyz = diff_z<ORDER, V, true>(ey, s1, q, n2), dxz = diff_z<ORDER, V, true>(ex, s0, q, n2);
     const fv<V> uy = axis_coeffs<V>(g, u1, 1), uz = axis_coeffs<V>(g, u1, 2);
-    h0 = pick_z<V, false>(XY || row_updated<false>(g, 0, q.i, q.j), q.k, n2, h0 - uy * dzy + uz * dyz, h0);
-    h1 = pick_z<V, false>(XY || row_updated<false>(g, 1, q.i, q.j), q.k, n2, h1 - uz * dxz + u1 * dzx, h1);
-    h2 = pick_z<V, true>(XY || row_updated<false>(g, 2, q.i, q.j), q.k, n2, h2 - u1 * dyx + uy * dxy, h2);
+    const fv<V> n0 = h0 - uy * dzy + uz * dyz, n1 = h1 - uz * dxz + u1 * dzx, nz = h2 - u1 * dyx + uy * dxy;
+    if (XY && q.zplain) {
+        h0 = n0;
+        h1 = n1;
+        h2 = nz;
+    } else {
+        h0 = pick_z<V, false>(XY || row_updated<false>(g, 0, q.i, q.j), q.k, n2, n0, h0);
+        h1 = pick_z<V, false>(XY || row_updated<false>(g, 1, q.i, q.j), q.k, n2, n1, h1);
+        h2 = pick_z<V, true>(XY || row_updated<false>(g, 2, q.i, q.j), q.k, n2, nz, h2);
+    }
     if constexpr (!XY) {
         {
             // x faces: (Hy, Ez), (Hz, Ey); y faces: (Hx, Ez), (Hz, Ex)
@@ -617,9 +629,17 @@ __device__ __forceinline__ void fwd_e_group(const Grid& g, const float* ca, cons
     const fv<V> uy = axis_coeffs<V>(g, u1, 1), uz = axis_coeffs<V>(g, u1, 2);
     const bool up[3] = {XY || row_updated<true>(g, 0, q.i, q.j), XY || row_updated<true>(g, 1, q.i, q.j),
                         XY || row_updated<true>(g, 2, q.i, q.j)};
-    e[0] = pick_z<V, true>(up[0], q.k, n2, u0 * e[0] + uy * dzy - uz * dyz, e[0]);
-    e[1] = pick_z<V, true>(up[1], q.k, n2, u0 * e[1] + uz * dxz - u1 * dzx, e[1]);
-    e[2] = pick_z<V, false>(up[2], q.k, n2, u0 * e[2] + u1 * dyx - uy * dxy, e[2]);
+    const fv<V> v0 = u0 * e[0] + uy * dzy - uz * dyz, v1 = u0 * e[1] + uz * dxz - u1 * dzx,
+                v2 = u0 * e[2] + u1 * dyx - uy * dxy;
+    if (XY && q.zplain) {
+        e[0] = v0;
+        e[1] = v1;
+        e[2] = v2;
+    } else {
+        e[0] = pick_z<V, true>(up[0], q.k, n2, v0, e[0]);
+        e[1] = pick_z<V, true>(up[1], q.k, n2, v1, e[1]);
+        e[2] = pick_z<V, false>(up[2], q.k, n2, v2, e[2]);
+    }
     if constexpr (!XY) {
         // x faces: (Ey, Hz), (Ez, Hy); y faces: (Ex, Hz), (Ez, Hx)
         row_face_apply<V, true>(g, 0, q, fx, cbv, dzx, dyx, e[1], e[2]);
@@ -1011,8 +1031,13 @@ __device__ __forceinline__ void adj_group(const Grid& g, const float* cu, const 
         const fv<V> a0 = channel_plus<EL>(0, 2) ? w0 + kz * l[1] : w0 - kz * l[1];
         const fv<V> a1 = channel_plus<EL>(1, 2) ? w1 + kz * l[0] : w1 - kz * l[0];
         // channel (x, z) targets y, channel (y, z) targets x
-        w0 = pick_z<V, EL>(XY || row_updated<EL>(g, 1, q.i, q.j), q.k, n2, a0, w0);
-        w1 = pick_z<V, EL>(XY || row_updated<EL>(g, 0, q.i, q.j), q.k, n2, a1, w1);
+        if (XY && q.zplain) {
+            w0 = a0;
+            w1 = a1;
+        } else {
+            w0 = pick_z<V, EL>(XY || row_updated<EL>(g, 1, q.i, q.j), q.k, n2, a0, w0);
+            w1 = pick_z<V, EL>(XY || row_updated<EL>(g, 0, q.i, q.j), q.k, n2, a1, w1);
+        }
     }
     stv<V>(s0, (unsigned)q.k, w0, q.dup);
     stv<V>(s1, (unsigned)q.k, w1, q.dup);
@@ -1051,9 +1076,15 @@ __device__ __forceinline__ void adj_group(const Grid& g, const float* cu, const 
     __syncthreads();
     gather_z<ORDER, V, EL>(q, n2, s0, s1, w0, w1, z0, z1);
     if (!EL) {
-        o[0] = pick_z<V, true>(XY || row_updated<true>(g, 0, q.i, q.j), q.k, n2, cav * o[0], o[0]);
-        o[1] = pick_z<V, true>(XY || row_updated<true>(g, 1, q.i, q.j), q.k, n2, cav * o[1], o[1]);
-        o[2] = pick_z<V, false>(XY || row_updated<true>(g, 2, q.i, q.j), q.k, n2, cav * o[2], o[2]);
+        if (XY && q.zplain) {
+            o[0] = cav * o[0];
+            o[1] = cav * o[1];
+            o[2] = cav * o[2];
+        } else {
+            o[0] = pick_z<V, true>(XY || row_updated<true>(g, 0, q.i, q.j), q.k, n2, cav * o[0], o[0]);
+            o[1] = pick_z<V, true>(XY || row_updated<true>(g, 1, q.i, q.j), q.k, n2, cav * o[1], o[1]);
+            o[2] = pick_z<V, false>(XY || row_updated<true>(g, 2, q.i, q.j), q.k, n2, cav * o[2], o[2]);
+        }
     }
     stv<V>(out.c[0], q.m, o[0] + y0 + z0, q.dup);
     stv<V>(out.c[1], q.m, o[1] + x1 + z1, q.dup);
