@@ -69,6 +69,8 @@ inline bool row_sweep_applies(const int N[3], const int pml[6], int order)
         if (hi < lo) return false;
         if (a == 2 && hi - lo + 1 < 32) return false;
         cells *= hi - lo + 1;
+        // the kernels look for a cell's face on its half of the axis
+        if (2 * pml[2 * a] > N[a] || 2 * pml[2 * a + 1] + 2 >= N[a]) return false;
     }
     return cells >= 65536 && N[2] <= 1024 && 1LL * N[0] * N[1] * N[2] < (1LL << 30);
 }

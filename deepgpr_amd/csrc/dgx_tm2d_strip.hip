@@ -1127,7 +1127,8 @@ StripMap map_order(const Tm2dGrid& g)
 
 bool strip_applies(int order, const Tm2dGrid& g)
 {
-    if (order > 4 || g.plane >= 1 << 30) return false;  // 32-bit byte offsets
+    // 32-bit byte offsets, and tiles along x and shots within a launch's 65535
+    if (order > 4 || g.plane >= 1 << 30 || g.NX > 1 << 20 || g.nshot > 65535) return false;
     // no face reaches the middle of its axis, and no strip of rows both faces
     return g.NX - g.pml[0] - g.pml[1] >= 12 && g.NY - g.pml[2] - g.pml[3] >= 4 && 2 * g.pml[0] + 9 < g.NX &&
            2 * g.pml[1] + 9 < g.NX && 2 * g.pml[2] + 2 < g.NY && 2 * g.pml[3] + 2 < g.NY;

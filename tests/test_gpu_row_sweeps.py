@@ -55,3 +55,17 @@ def test_row_sweeps_match_oracle_bitwise(oracle_built, cuda_device, case):
     assert not bad, bad
     assert np.array_equal(gpu["E_saved"], cpu["E_saved"])
     assert np.array_equal(gpu["R_saved"], cpu["R_saved"])
+
+
+@pytest.mark.parametrize("shape,pml", [((64, 80, 96), (36, 4, 4, 4, 4, 4)), ((80, 66, 96), (4, 4, 5, 36, 4, 3)),
+                                       ((70, 70, 100), (4, 4, 4, 4, 56, 3))])
+def test_faces_beyond_the_middle_match_oracle(oracle_built, cuda_device, shape, pml):
+    """A CPML that reaches past the middle of its axis."""
+    h = oracle_built
+    print(f"[gpu row sweeps] faces beyond the middle {shape} {pml}", flush=True)
+    p = h.make_problem(*shape, order=2, nt=4, nshot=1, nsrc=2, nrx=4, seed=29, pml=pml, d=(0.02, 0.02, 0.02))
+    p.src_loc[0, 0] = [shape[0] // 2, shape[1] // 2, shape[2] // 2]
+    cpu = h.run_cpu(p, "oracle")
+    gpu = h.run_gpu(p, api="dgx")
+    bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
+    assert not bad, bad
