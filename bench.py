@@ -122,11 +122,13 @@ def model_bytes_per_cell(w, args):
     return fwd, adj
 
 
-def kernel_bytes(kernel: str, w, args) -> float:
+def kernel_bytes(kernel: str, w, args, steps: float = 1.0) -> float:
     """Algorithmic bytes of ONE launch of a kernel (one time step, all shots of
-    one call). The fused 2D TM kernels carry the per-cell model above times
-    the cells they advance; the gradient accumulators belong to the reduction
-    kernel while it is separate. The split kernels carry their own share of
+    one call; `steps` time steps for the strip kernels, which read and write
+    the state once a launch and the Ez history once a step). The one-step 2D TM
+    kernels carry the per-cell model above times the cells they advance; the
+    gradient accumulators belong to the reduction kernel while it is separate.
+    The split kernels carry their own share of
     the compulsory loads/stores."""
     shots = args.shots_per_call or w.source_location.shape[0]
     ext = w.extended_cells()
@@ -136,6 +138,8 @@ def kernel_bytes(kernel: str, w, args) -> float:
     comps, hist_b, frames = _history_terms(w, args)
     fwd, adj = model_bytes_per_cell(w, args)
     acc_b = 2 * 2 * (8.0 if args.accumulator == "float64" else 4.0) / w.sampling_interval
+    if kernel in ("tm_strip_fwd", "tm_strip_adj"):
+        return cells * (32.0 + steps * hist_b / w.sampling_interval) + 8 * (pe + ph)
     if kernel == "tm_step_fwd":
         return fwd * cells
     if kernel == "tm_step_adj":
@@ -167,8 +171,9 @@ def kernel_bytes(kernel: str, w, args) -> float:
 # accumulator, shots per call): traffic depends on all of them. The commands
 # and per-kernel tables are in the profiles/*.md file named with each entry.
 MEASURED_TRAFFIC = {
-    ("c2", "tm_step_adj", "float32", "float64", 20): (121.9e6, "profiles/c2_fwi_2d_o4_tm_step_kernels.md"),
-    ("c2", "tm_step_fwd", "float32", "float64", 20): (90.4e6, "profiles/c2_fwi_2d_o4_tm_step_kernels.md"),
+    ("c3", "adj_e", "float32", "float64", 1): (1334.7e6, "profiles/c3_layered_3d_o4_kernels.md"),
+    ("c2", "tm_strip_adj", "float32", "float64", 20): (249.2e6, "profiles/c2_fwi_2d_o4_strip_kernels.md"),
+    ("c2", "tm_strip_fwd", "float32", "float64", 20): (162.1e6, "profiles/c2_fwi_2d_o4_strip_kernels.md"),
 }
 
 
@@ -359,7 +364,7 @@ def main():
             _, dom = ranked[0]
             tot, cnt = kernels[dom]
             avg_s = tot / cnt / 1e3
-            bytes_launch = kernel_bytes(dom, w, args)
+            bytes_launch = kernel_bytes(dom, w, args, w.nt / cnt)
             achieved = bytes_launch / avg_s / 1e9
             measured = MEASURED_TRAFFIC.get((args.workload, dom, args.storage, args.accumulator, chunk))
             roofline = {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,

@@ -22,7 +22,7 @@
 // against 58, 68 and 179 now; order 2 on 165 x 141 x 189, 45, 51 and 101 against
 // 42, 45 and 98. What bounds them now is the chain of a wavefront (loads, row
 // exchange, z-CPML loads, stores) at 4 wavefronts a SIMD and, in the adjoint,
-// the vector instructions (62 % of the cycles), not the bytes.
+// the vector instructions (42 % of the cycles), not the bytes.
 //
 // Four wavefronts need at most 128 registers a lane, so what only the end of a
 // sweep uses is loaded there: with the old fields, cb and the adjoint's outputs
