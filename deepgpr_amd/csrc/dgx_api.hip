@@ -1700,17 +1700,25 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
         tgrad.nsrc = P->nsource;
     }
     // Two buffers: a launch writes one while it sums the other (the previous
-    // saved step). The strip kernels write up to strip_saves saved steps of
-    // several shots and the sum kernel adds them; their buffers take no more
-    // than two did, or 32 MiB.
+    // saved step). The strip kernels hold up to strip_saves saved steps of
+    // several shots before the sum kernel adds them: a sum of few cells is a
+    // launch and its latency, whose cost the steps share (5 shots of 342 x 264,
+    // 400 steps, a gradient: 11.1 ms with a sum after each launch, 9.7 now).
+    // Their buffers take no more than two did, or 32 MiB: 20 shots of 441 x 241
+    // keep two steps, whose sum is bound by its bytes. A sum of more than 32
+    // steps would be a longer chain and no fewer bytes.
     const long long terms_len = 2 * (long long)g.nshot * pl.box.cells;
-    const int strip_saves =
-        strips ? (int)std::min<long long>(stm.sh.steps, std::max<long long>(2, (8LL << 20) / std::max(terms_len, 1LL)))
-               : 2;
+    int strip_saves = 2;
+    if (strips)
+        strip_saves = (int)std::min<long long>(32, std::max<long long>(2, (8LL << 20) / std::max(terms_len, 1LL)));
     if (fused && want_mat && !(strips && g.nshot == 1) &&
         !d_terms.alloc((size_t)strip_saves * terms_len * sizeof(float))) {
-        set_error("backward: out of device memory for per-shot gradient terms");
-        return -1;
+        (void)hipGetLastError();  // out of memory: two may still fit
+        strip_saves = 2;
+        if (!d_terms.alloc((size_t)strip_saves * terms_len * sizeof(float))) {
+            set_error("backward: out of device memory for per-shot gradient terms");
+            return -1;
+        }
     }
 
     // CPML weight scratch, shaped like the psi arrays
@@ -1888,21 +1896,29 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
         sg.src_vals = tgrad.src_vals;
         sg.nsrc = tgrad.nsrc;
         sg.geo = geo;
+        int held = 0;  // saved steps whose terms wait for their sum
+        auto sum_held = [&] {
+            if (held > 0)
+                TIMED(tmr, kKTmGradReduce,
+                      launch_tm_grad_reduce(tms.g, pl.box, (const float*)d_terms.p, held, terms_len, mg.want_eps,
+                                            mg.want_sig, geps, gsig, fp64, stream));
+            held = 0;
+        };
         for (int it = nt - 1; it >= 0;) {
             int nsub = std::min(stm.sh.steps, it + 1);
             // saved steps among it - nsub + 1 .. it: multiples of S
             auto saves = [&](int n) { return want_mat ? it / sg.S - (it - n + sg.S) / sg.S + 1 : 0; };
             if (g.nshot > 1)
                 while (saves(nsub) > strip_saves) --nsub;
+            if (held + saves(nsub) > strip_saves) sum_held();
+            sg.terms = (float*)d_terms.p + held * terms_len;
             TIMED(tmr, kKTmStripAdj,
                   launch_tm_strip_adj(pl.order, tms.g, tms.f, tms.pp, stm, tsrc, tax, sg, it, nsub, fp64, stream));
             tms.flip();
-            if (g.nshot > 1 && saves(nsub) > 0)
-                TIMED(tmr, kKTmGradReduce,
-                      launch_tm_grad_reduce(tms.g, pl.box, sg.terms, saves(nsub), terms_len, mg.want_eps, mg.want_sig,
-                                            geps, gsig, fp64, stream));
+            if (g.nshot > 1) held += saves(nsub);
             it -= nsub;
         }
+        sum_held();
     }
     for (int it = strips ? -1 : nt - 1; it >= 0; --it) {
         if (fused) {

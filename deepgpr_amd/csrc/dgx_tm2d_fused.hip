@@ -186,7 +186,26 @@ __global__ __launch_bounds__(256) void k_tm_grad_reduce(Tm2dGrid g, Box b, const
     ACC* acc = (sig ? gsig : geps) + terms_out(g, b, h);
     const float* t = terms + (sig ? (long long)g.nshot * b.cells : 0) + h;
     ACC sum = *acc;
-    for (int k = 0; k < steps; ++k) sum += sum_shots<ACC>(t + k * terms_len, b.cells, g.nshot);
+    int k = 0;
+    if (g.nshot <= 8)  // the loads of two steps before their adds: few shots wait for memory, not for bytes
+        for (; k + 2 <= steps; k += 2) {
+            float x[2][8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const float* v = t + k * terms_len + min(q, g.nshot - 1) * b.cells;
+                x[0][q] = v[0];
+                x[1][q] = v[terms_len];
+            }
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                ACC a = 0;
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    if (q < g.nshot) a += (ACC)x[p][q];
+                sum += a;
+            }
+        }
+    for (; k < steps; ++k) sum += sum_shots<ACC>(t + k * terms_len, b.cells, g.nshot);
     *acc = sum;
 }
 

@@ -81,6 +81,24 @@ def test_strips_match_oracle_bitwise(oracle_built, cuda_device, monkeypatch, cas
     assert np.array_equal(gpu["R_saved"], cpu["R_saved"])
 
 
+
+@pytest.mark.parametrize("case", [(19, 23, 2, 75, 2, 1, "f32", 2), (43, 57, 4, 71, 5, 2, "bf16", 3),
+                                  (30, 41, 4, 40, 9, 1, "e_only", 2), (47, 38, 2, 101, 8, 3, "f16", 3)],
+                         ids=lambda c: f"{c[0]}x{c[1]}-o{c[2]}-nt{c[3]}-n{c[4]}")
+def test_held_material_terms_are_summed_in_order(oracle_built, cuda_device, monkeypatch, case):
+    """Terms of several launches wait for one sum: more saved steps than the buffer holds, odd numbers of them left,
+    shots below, at and above the eight that the sum loads at once."""
+    h = oracle_built
+    monkeypatch.delenv("DEEPGPR_AMD_TM2D_TILE_ROWS", raising=False)
+    print(f"[gpu strips] held terms {case}", flush=True)
+    p = _problem(h, case + ((4, 3, 5, 4), (0.02, 0.018), True))
+    cpu = h.run_cpu(p, "oracle")
+    p.storage_type |= TM2D
+    gpu = h.run_gpu(p, api="dgx")
+    bad = h.bitwise_diff(gpu, cpu, h.KEYS_FWD + ("g_src", "g_eps", "g_sig"))
+    assert not bad, bad
+
+
 def _request(rid, shape, nt, order, nshot, gradient, seed):
     from deepgpr_amd.serving import SolveRequest
     gen = torch.Generator().manual_seed(seed)
