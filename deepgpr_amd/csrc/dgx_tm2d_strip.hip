@@ -1068,7 +1068,14 @@ namespace {
 // Hence the rule of map_order: shape 0 as long as each of its workgroups (1024
 // threads) has a compute unit to itself, shape 1 as long as its workgroups (512
 // threads, two a compute unit) are all resident at once, then shape 2, whose
-// larger tile has the smaller margin.
+// larger tile has the smaller margin. Before them comes shape 3, which is shape 0
+// with more steps a launch and a margin that leaves 8 rows of 32: where its
+// workgroups have a compute unit each as well, the margin costs no time and the
+// launches are fewer. 600 steps, forward and gradient in ms, one shot, shape 0
+// and shape 3: order 2, 121 x 121, 2.01 and 4.30 against 1.87 and 3.99; order 4,
+// 3.01 and 6.47 against 2.85 and 5.89; 221 x 221, order 2, 2.05 and 4.48 against
+// 1.98 and 4.15, order 4, 3.06 and 6.62 against 2.80 and 5.99. 10 steps at order 2:
+// 1.93 and 4.15.
 template <int ORDER, int SIZE>
 struct Shapes;
 template <>
@@ -1095,6 +1102,14 @@ template <>
 struct Shapes<4, 2> {
     static constexpr int KR = 4, NW = 16, T = 2;
 };
+template <>
+struct Shapes<2, 3> {
+    static constexpr int KR = 2, NW = 16, T = 12;
+};
+template <>
+struct Shapes<4, 3> {
+    static constexpr int KR = 2, NW = 16, T = 4;
+};
 template <int ORDER, int SIZE>
 StripShape shape_of()
 {
@@ -1112,11 +1127,14 @@ void launch_order(const dim3& grid, const StripArgs& a, hipStream_t st)
 {
     if (a.sm.sh.size == 0) launch_shape<ORDER, 0>(grid, a, st);
     else if (a.sm.sh.size == 1) launch_shape<ORDER, 1>(grid, a, st);
-    else launch_shape<ORDER, 2>(grid, a, st);
+    else if (a.sm.sh.size == 2) launch_shape<ORDER, 2>(grid, a, st);
+    else launch_shape<ORDER, 3>(grid, a, st);
 }
 template <int ORDER>
 StripMap map_order(const Tm2dGrid& g)
 {
+    const StripMap deep = make_strip_map(shape_of<ORDER, 3>(), g.NX, g.NY);
+    if ((long long)deep.tiles * g.nshot <= 256) return deep;
     const StripMap small = make_strip_map(shape_of<ORDER, 0>(), g.NX, g.NY);
     if ((long long)small.tiles * g.nshot <= 256) return small;
     const StripMap mid = make_strip_map(shape_of<ORDER, 1>(), g.NX, g.NY);
@@ -1163,7 +1181,8 @@ void launch_adj_order(const dim3& grid, const StripAdjArgs& a, bool fp64, hipStr
 {
     if (a.sm.sh.size == 0) launch_adj_shape<ORDER, 0>(grid, a, fp64, st);
     else if (a.sm.sh.size == 1) launch_adj_shape<ORDER, 1>(grid, a, fp64, st);
-    else launch_adj_shape<ORDER, 2>(grid, a, fp64, st);
+    else if (a.sm.sh.size == 2) launch_adj_shape<ORDER, 2>(grid, a, fp64, st);
+    else launch_adj_shape<ORDER, 3>(grid, a, fp64, st);
 }
 }  // namespace
 

@@ -29,6 +29,10 @@ CASES = [
     (64, 105, 2, 8, 43, 2, "f32", 3, (6, 9, 10, 5), (0.02, 0.019), True),
     (52, 62, 2, 9, 1, 1, "e_only", 3, (7, 6, 5, 8), (0.02, 0.02), False),
     (46, 38, 4, 7, 3, 1, "f16_e", 3, (6, 5, 7, 3), (0.02, 0.018), True),
+    (61, 209, 2, 11, 7, 1, "e_only", 2, (10, 10, 9, 10), (0.02, 0.018), True),
+    (81, 104, 4, 7, 9, 1, "f32", 3, (9, 10, 8, 10), (0.02, 0.02), False),
+    (64, 81, 2, 25, 4, 1, "f32", 2, (10, 9, 12, 11), (0.02, 0.02), True),
+    (41, 83, 4, 9, 6, 2, "bf16", 3, (3, 6, 7, 4), (0.02, 0.017), False),
     (300, 700, 2, 9, 1, 2, "f32", 3, (10, 7, 9, 10), (0.02, 0.02), True),
     (251, 731, 4, 5, 1, 1, "e_only", 2, (10, 7, 9, 10), (0.02, 0.021), False),
 ]
