@@ -1756,7 +1756,7 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
 
     // row sweeps: second copies of the lambda psi arrays of the x and y faces; a
     // half step reads its neighbours' old ones while it writes its own (those
-    // of the z faces are read at their own cells alone)
+    // of the z faces only serve the thread that advances them)
     DevBuf d_psi;
     Cpml psi_set[2][2] = {{pl.cpe, pl.cph}, {pl.cpe, pl.cph}};  // [copy][E, H]
     CopySpans psi_copy{};

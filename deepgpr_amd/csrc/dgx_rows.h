@@ -205,6 +205,14 @@ DGX_HD bool row_thread(const RowMap& m, const RowKind& kd, int V, int t, int nj,
     return false;
 }
 
+// Whether element e of a group (its cell k + e) comes from the group's own
+// registers in a z-stencil, not from the row buffer, which every owner fills
+// before the barrier. The adjoint's z weights are formed from CPML auxiliaries
+// that their owner advances in place, so a cell of the group before (e < dup)
+// is right in the buffer alone: the thread before it may be in another
+// wavefront and have advanced the auxiliary already.
+DGX_HD bool row_own_element(int e, int dup, int V) { return e >= dup && e < V; }
+
 // Workgroup of a shot that owns row (i, j).
 inline int row_block_of(const RowMap& m, int i, int j)
 {

@@ -931,8 +931,9 @@ __device__ __forceinline__ void psi_advance(const Grid& g, int a, const fv<V> (&
 }
 
 // Channels (x, z) and (y, z): the weights of the group's own cells (w0, w1,
-// with the z-CPML terms, whose auxiliaries advance here) and, in sw, those of
-// the rows of the workgroup.
+// with the z-CPML terms, whose auxiliaries have advanced by now) and, in s0 and
+// s1, those of the row, which its moved-back last group takes for the cells of
+// the group before it (row_own_element).
 template <int ORDER, int V, bool EL>
 __device__ __forceinline__ void gather_z(const Group& q, int n, const float* s0, const float* s1, const fv<V>& w0,
                                          const fv<V>& w1, fv<V>& g0, fv<V>& g1)
@@ -950,6 +951,14 @@ __device__ __forceinline__ void gather_z(const Group& q, int n, const float* s0,
     for (int e = 0; e < V; ++e) {
         a0[L + e] = w0[e];
         a1[L + e] = w1[e];
+    }
+    if (q.dup > 0) {
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            if (!row_own_element(e, q.dup, V)) {
+                a0[L + e] = s0[q.k + e];
+                a1[L + e] = s1[q.k + e];
+            }
     }
 #pragma unroll
     for (int e = 0; e < U; ++e) {
@@ -993,7 +1002,8 @@ __device__ __forceinline__ void gather_z(const Group& q, int n, const float* s0,
 }
 
 // The z-CPML terms of the group's own channel weights, and its auxiliaries
-// advanced (they are only read at their own cells, so in place).
+// advanced in place: the terms of cells that another thread owns may come from
+// advanced ones and are not used (row_own_element).
 template <int V, bool EL>
 __device__ __forceinline__ void z_weights(const Grid& g, const Group& gr, const ZFace<V>& zf, const fv<V>& lx,
                                           const fv<V>& ly, fv<V>& w0, fv<V>& w1)

@@ -69,3 +69,21 @@ def test_faces_beyond_the_middle_match_oracle(oracle_built, cuda_device, shape, 
     gpu = h.run_gpu(p, api="dgx")
     bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
     assert not bad, bad
+
+
+@pytest.mark.parametrize("shape,order,pz,nt", [((60, 58, 142), 4, 20, 7), ((60, 60, 91), 4, 21, 6),
+                                               ((60, 60, 63), 2, 6, 7), ((62, 60, 67), 2, 10, 6)])
+def test_split_row_ends_match_oracle(oracle_built, cuda_device, shape, order, pz, nt):
+    """Rows whose last two groups overlap and lie in two wavefronts of a workgroup (tests/native/row_window_check.cpp)."""
+    h = oracle_built
+    print(f"[gpu row sweeps] split row ends {shape} {order} {pz}", flush=True)
+    p = h.make_problem(*shape, order=order, nt=nt, nshot=2, nsrc=2, nrx=6, seed=43, pml=(4, 4, 4, 4, pz, pz),
+                       d=(0.02, 0.017, 0.015))
+    for s in range(2):
+        p.src_loc[s, 0] = [shape[0] // 2, shape[1] // 2, shape[2] - 4]
+        for r in range(6):
+            p.rx_loc[s, r] = [10 + 8 * r, 5 + 9 * r, shape[2] - 2 - r]
+    cpu = h.run_cpu(p, "oracle")
+    gpu = h.run_gpu(p, api="dgx")
+    bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
+    assert not bad, bad
