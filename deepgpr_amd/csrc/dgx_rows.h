@@ -52,6 +52,23 @@ DGX_HD void row_plain_range(int n, int plo, int phi, int R, int& lo, int& hi)
     if (phi > 0 && n - 2 - phi - R < hi) hi = n - 2 - phi - R;
 }
 
+// The face of an axis of n cells that a thread of the row sweeps looks at: the
+// one on the side of its cell c (along z, of its first cell).
+DGX_HD bool row_high_side(int c, int n) { return 2 * c > n; }
+
+// Cells beyond its own for which a thread relies on that face: the taps of the
+// adjoint along x and y (radius 2 at order 4), and the others of its group along z.
+constexpr int kRowReach = 3;
+
+// A face of width p, on the low or the high side of an axis of n cells, that is
+// in no thread's reach on the other side: its cells are 0 .. p or n - 1 - p .. n - 2.
+inline bool row_face_fits(int n, int p, bool high)
+{
+    if (p <= 0) return true;
+    const int last_low = n / 2;  // the last cell for which row_high_side is false
+    return high ? last_low + kRowReach < n - 1 - p : last_low + 1 - kRowReach > p;
+}
+
 // The row sweeps take solves of order 2 and 4 on grids with a plain interior
 // that is worth it: at least 65536 cells plain for every order, in rows of at
 // least 32 of them and at most 1024 cells (a row fits a workgroup of 512
@@ -69,8 +86,7 @@ inline bool row_sweep_applies(const int N[3], const int pml[6], int order)
         if (hi < lo) return false;
         if (a == 2 && hi - lo + 1 < 32) return false;
         cells *= hi - lo + 1;
-        // the kernels look for a cell's face on its half of the axis
-        if (2 * pml[2 * a] > N[a] || 2 * pml[2 * a + 1] + 2 >= N[a]) return false;
+        if (!row_face_fits(N[a], pml[2 * a], false) || !row_face_fits(N[a], pml[2 * a + 1], true)) return false;
     }
     return cells >= 65536 && N[2] <= 1024 && 1LL * N[0] * N[1] * N[2] < (1LL << 30);
 }

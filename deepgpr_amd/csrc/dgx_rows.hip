@@ -227,8 +227,9 @@ __device__ __forceinline__ T choose(bool c, T a, T b)
     return c ? a : b;
 }
 
-// The face of axis a on the side of coordinate c: the cells [lo, hi] of its
-// region and their profile index, hi - c on the low side, c - lo on the high.
+// The face of axis a on the side of coordinate c (row_face_fits: the only one in
+// the thread's reach): the cells [lo, hi] of its region and their profile index,
+// hi - c on the low side, c - lo on the high.
 struct Side {
     bool high;
     int p, lo, hi;
@@ -241,7 +242,7 @@ __device__ __forceinline__ Side side_of(const Grid& g, int a, int c)
 {
     Side o;
     const int n = g.N[a];
-    o.high = 2 * c > n;
+    o.high = row_high_side(c, n);
     o.p = choose(o.high, g.pml[2 * a + 1], g.pml[2 * a]);
     o.lo = o.high ? n - 1 - o.p : (EL ? 1 : 0);
     o.hi = o.high ? n - 2 : (EL ? o.p : o.p - 1);

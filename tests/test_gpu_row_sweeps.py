@@ -87,3 +87,19 @@ def test_split_row_ends_match_oracle(oracle_built, cuda_device, shape, order, pz
     gpu = h.run_gpu(p, api="dgx")
     bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
     assert not bad, bad
+
+
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("shape,pml", [((80, 72, 84), (4, 38, 4, 4, 4, 4)), ((74, 81, 84), (4, 4, 38, 0, 3, 4)),
+                                       ((72, 72, 84), (4, 4, 4, 4, 3, 40)), ((72, 72, 84), (4, 4, 4, 4, 5, 36)),
+                                       ((81, 80, 90), (36, 3, 0, 35, 4, 4))])
+def test_faces_close_to_the_middle_match_oracle(oracle_built, cuda_device, shape, pml, order):
+    """A CPML that ends within a few cells of the middle of its axis, one side or the other of what row sweeps take."""
+    h = oracle_built
+    print(f"[gpu row sweeps] faces close to the middle {shape} {pml} {order}", flush=True)
+    p = h.make_problem(*shape, order=order, nt=4, nshot=1, nsrc=2, nrx=4, seed=31, pml=pml, d=(0.02, 0.02, 0.02))
+    p.src_loc[0, 0] = [shape[0] // 2, shape[1] // 2, shape[2] // 2]
+    cpu = h.run_cpu(p, "oracle")
+    gpu = h.run_gpu(p, api="dgx")
+    bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
+    assert not bad, bad
