@@ -149,3 +149,28 @@ def test_batch_of_strips_equals_one_step_launches(cuda_device, monkeypatch):
             if r.gradient:
                 assert torch.equal(res[1], a.grad_eps_r), (strips, r.rid)
                 assert torch.equal(res[2], a.grad_sigma), (strips, r.rid)
+
+
+@pytest.mark.parametrize("order", [2, 4])
+def test_signs_of_zeros_equal_the_one_step_kernels(oracle_built, cuda_device, monkeypatch, order):
+    """Fields and auxiliaries of zeros of either sign: quotients of -0 by the grid spacing keep their sign, so both
+    kernels leave the same bits, those of the zeros included."""
+    h = oracle_built
+    monkeypatch.delenv("DEEPGPR_AMD_TM2D_TILE_ROWS", raising=False)
+    print(f"[gpu strips] signs of zeros, order {order}", flush=True)
+    p = _problem(h, (57, 71, order, 3, 2, 1, "f32", 2, (9, 8, 7, 10), (0.02, 0.017), False))
+    rng = np.random.default_rng(order)
+    for arrs in (p.E0, p.H0, p.phi0):
+        for k, a in enumerate(arrs):
+            arrs[k] = np.where(rng.random(a.shape) < 0.5, np.float32(-0.0), np.float32(0.0))
+    for arrs, idx in ((p.E0, (0, 1)), (p.H0, (2,)), (p.phi0, INACTIVE_PHI)):
+        for k in idx:
+            arrs[k] = np.zeros_like(arrs[k])
+    p.wave = np.zeros_like(p.wave)
+    p.storage_type |= TM2D
+    strips = h.run_gpu(p, backward=False, api="dgx")
+    monkeypatch.setenv("DEEPGPR_AMD_TM2D_STRIPS", "0")
+    steps = h.run_gpu(p, backward=False, api="dgx")
+    for key in ("E", "H", "phi"):
+        for k, (a, b) in enumerate(zip(strips[key], steps[key])):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (key, k)
