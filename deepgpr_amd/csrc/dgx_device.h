@@ -439,11 +439,11 @@ __device__ __forceinline__ float gather_fwd_sel(WF wf, int c, int n)
 // x[q] / d, correctly rounded, for n values at once: with y the correctly
 // rounded 1 / d, q = x y and r = x - q d (exact in one fused multiply-add),
 // q + r y rounds to the quotient (Markstein, "Computation of elementary
-// functions on the IBM RISC System/6000 processor", 1990); a zero takes its sign
-// from x, which the sum of zeros loses. That needs r not to
-// underflow and nothing to overflow, so values outside 2^-90 .. 2^90 (zeros
-// aside), infinities, NaN and spacings outside 2^-30 .. 2^30 take the division
-// proper.
+// functions on the IBM RISC System/6000 processor", 1990). As -(q d - x), r is
+// -0 where it is zero, so that q + r y keeps the sign of a q of zero, which x - q d
+// = +0 would lose for -0 / d. That needs r not to underflow and nothing to
+// overflow, so values outside 2^-90 .. 2^90 (zeros aside), infinities, NaN and
+// spacings outside 2^-30 .. 2^30 take the division proper.
 struct Spacing {
     float d, y, big;
 };
@@ -462,7 +462,7 @@ __device__ __forceinline__ void div_all(const float (&x)[N], const Spacing& sp, 
 #pragma unroll
     for (int q = 0; q < N; ++q) {
         const float t = x[q] * y;
-        out[q] = __builtin_copysignf(__builtin_fmaf(__builtin_fmaf(-t, d, x[q]), y, t), x[q]);
+        out[q] = __builtin_fmaf(-__builtin_fmaf(t, d, -x[q]), y, t);
         // an unordered compare later takes a NaN; fmaxf would drop it
         big = big + __builtin_fabsf(x[q]);
         small = min(small, (__float_as_uint(x[q]) << 1) - 1u);
