@@ -941,25 +941,41 @@ void tm_receiver_groups(const Tm2dGrid& g, int order, const std::vector<int>& go
     for (size_t k = 1; k < off.size(); ++k) off[k] += off[k - 1];
 }
 
-// Entries of strip lists: grouped by (tile, shot), in input order within one.
+// Entries (list, entry) grouped by list, in input order within one: ent[off[k] ..
+// off[k + 1]) are those of list k.
 template <typename E>
-void strip_lists(std::vector<std::pair<long long, E>>& tmp, long long lists, std::vector<int>& off, std::vector<E>& ent)
+void group_lists(const std::vector<std::pair<long long, E>>& tmp, long long lists, std::vector<int>& off,
+                 std::vector<E>& ent)
 {
-    std::stable_sort(tmp.begin(), tmp.end(),
-                     [](const std::pair<long long, E>& a, const std::pair<long long, E>& b) { return a.first < b.first; });
     off.assign((size_t)lists + 1, 0);
-    ent.clear();
-    for (const auto& e : tmp) {
-        off[(size_t)e.first + 1] += 1;
-        ent.push_back(e.second);
-    }
+    for (const auto& e : tmp) off[(size_t)e.first + 1] += 1;
     for (size_t k = 1; k < off.size(); ++k) off[k] += off[k - 1];
+    ent.resize(tmp.size());
+    std::vector<int> next(off.begin(), off.end() - 1);
+    for (const auto& e : tmp) ent[(size_t)next[(size_t)e.first]++] = e.second;
 }
 
 // Points of every shot (loc: nshot x n x 3) as (staged index, point) entries of
-// the tile that owns the cell or, with `margin`, of every tile that stages it.
-void strip_points(const StripMap& m, int nshot, const std::vector<int>& loc, int n, bool margin, std::vector<int>& off,
-                  std::vector<int2>& ent)
+// the tile that owns the cell: one list a (tile, shot).
+void strip_owned_points(const StripMap& m, int nshot, const std::vector<int>& loc, int n, std::vector<int>& off,
+                        std::vector<int2>& ent)
+{
+    std::vector<std::pair<long long, int2>> tmp;
+    tmp.reserve((size_t)nshot * n);
+    for (int s = 0; s < nshot; ++s)
+        for (int k = 0; k < n; ++k) {
+            const int* L = &loc[((size_t)s * n + k) * 3];
+            const int a = L[0] / m.orow, b = L[1] / m.ocol;
+            tmp.push_back({a * m.ntj + b + (long long)m.tiles * s, make_int2(strip_local(m, a, b, L[0], L[1]), k)});
+        }
+    group_lists(tmp, (long long)m.tiles * nshot, off, ent);
+}
+
+// Points as entries of the wavefront that stages the cell in the tile that owns
+// it or, with `margin`, in every tile that stages it: one list a (tile, shot,
+// wavefront), by lane, the points of a lane in input order.
+void strip_wave_points(const StripMap& m, int nshot, const std::vector<int>& loc, int n, bool margin,
+                       std::vector<int>& off, std::vector<int2>& ent)
 {
     std::vector<std::pair<long long, int2>> tmp;
     for (int s = 0; s < nshot; ++s)
@@ -971,15 +987,22 @@ void strip_points(const StripMap& m, int nshot, const std::vector<int>& loc, int
                 strip_tiles(L[1], m.ocol, m.sh.halo, 64, m.ntj, b0, b1);
             }
             for (int a = a0; a <= a1; ++a)
-                for (int b = b0; b <= b1; ++b)
-                    tmp.push_back({a * m.ntj + b + (long long)m.tiles * s,
-                                   make_int2(strip_local(m, a, b, L[0], L[1]), k)});
+                for (int b = b0; b <= b1; ++b) {
+                    const int local = strip_local(m, a, b, L[0], L[1]);
+                    tmp.push_back({(a * m.ntj + b + (long long)m.tiles * s) * m.sh.waves + strip_wave(m, local),
+                                   make_int2(local, k)});
+                }
         }
-    strip_lists(tmp, (long long)m.tiles * nshot, off, ent);
+    group_lists(tmp, (long long)m.tiles * nshot * m.sh.waves, off, ent);
+    for (size_t q = 0; q + 1 < off.size(); ++q)
+        if (off[q + 1] - off[q] > 1)
+            std::stable_sort(ent.begin() + off[q], ent.begin() + off[q + 1],
+                             [](const int2& a, const int2& b) { return (a.x & 63) < (b.x & 63); });
 }
 
 // Receiver groups (as tm_receiver_groups takes them) listed for every (tile,
-// shot) that stages the cell: (staged index, first member, member count, 0).
+// shot, wavefront) that stages the cell: (staged index, first member, member
+// count, 0).
 void strip_groups(const StripMap& m, int nshot, int ny, const std::vector<int>& goff, const std::vector<int>& gshot,
                   const std::vector<long long>& gcell, std::vector<int>& off, std::vector<int4>& grp)
 {
@@ -990,11 +1013,13 @@ void strip_groups(const StripMap& m, int nshot, int ny, const std::vector<int>& 
         strip_tiles(i, m.orow, m.sh.halo, m.sh.rows, m.nti, a0, a1);
         strip_tiles(j, m.ocol, m.sh.halo, 64, m.ntj, b0, b1);
         for (int a = a0; a <= a1; ++a)
-            for (int b = b0; b <= b1; ++b)
-                tmp.push_back({a * m.ntj + b + (long long)m.tiles * gshot[q],
-                               make_int4(strip_local(m, a, b, i, j), goff[q], goff[q + 1] - goff[q], 0)});
+            for (int b = b0; b <= b1; ++b) {
+                const int local = strip_local(m, a, b, i, j);
+                tmp.push_back({(a * m.ntj + b + (long long)m.tiles * gshot[q]) * m.sh.waves + strip_wave(m, local),
+                               make_int4(local, goff[q], goff[q + 1] - goff[q], 0)});
+            }
     }
-    strip_lists(tmp, (long long)m.tiles * nshot, off, grp);
+    group_lists(tmp, (long long)m.tiles * nshot * m.sh.waves, off, grp);
 }
 
 // Receiver groups of one call: one per (shot, cell), members in receiver
@@ -1157,7 +1182,7 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
     std::vector<int> boff((size_t)nblocks + 1, 0);
     std::vector<int2> ents;
     if (inject && strips) {
-        strip_points(stm, g.nshot, hsloc, P->nsource, true, boff, ents);
+        strip_wave_points(stm, g.nshot, hsloc, P->nsource, true, boff, ents);
     } else if (inject && fused) {
         tm_source_lists(tg, hsloc, P->nsource, boff, ents);
     } else if (inject) {
@@ -1239,7 +1264,7 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
     if (fused_rx) {
         std::vector<int> roff;
         std::vector<int2> rent;
-        if (strips) strip_points(stm, g.nshot, hrloc, P->nreceiver, false, roff, rent);
+        if (strips) strip_owned_points(stm, g.nshot, hrloc, P->nreceiver, roff, rent);
         else tm_receiver_lists(tg, hrloc, P->nreceiver, roff, rent);
         if (!upload(d_roff, roff, stream) || !upload(d_rent, rent, stream)) {
             set_error("forward: out of device memory for receiver lists");
@@ -1686,7 +1711,7 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
     if (fused && want_src) {
         std::vector<int> soff;
         std::vector<int2> sent;
-        if (strips) strip_points(stm, g.nshot, hsloc, P->nsource, false, soff, sent);
+        if (strips) strip_wave_points(stm, g.nshot, hsloc, P->nsource, false, soff, sent);
         else tm_source_lists(tg, hsloc, P->nsource, soff, sent);
         if (!upload(d_soff, soff, stream) || !upload(d_sent, sent, stream) ||
             !d_svals.alloc((size_t)nt * g.nshot * P->nsource * sizeof(float))) {
@@ -2293,8 +2318,8 @@ int batch_add(Batch* b, const dgx_solve* P, const dgx_solve* G, hipStream_t stre
     I.strip = g.nshot == 1 && tm2d_strips() && strip_applies(pl.order, tg);
     const StripMap stm = I.strip ? strip_batch_map(pl.order, tg) : StripMap{};
     if (I.strip) {
-        strip_points(stm, 1, hsloc, P->nsource, true, soff, sent);
-        strip_points(stm, 1, hrloc, P->nreceiver, false, roff, rent);
+        strip_wave_points(stm, 1, hsloc, P->nsource, true, soff, sent);
+        strip_owned_points(stm, 1, hrloc, P->nreceiver, roff, rent);
     } else {
         tm_source_lists(tg, hsloc, P->nsource, soff, sent);
         tm_receiver_lists(tg, hrloc, P->nreceiver, roff, rent);

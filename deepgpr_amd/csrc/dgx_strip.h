@@ -16,6 +16,7 @@ struct StripShape {
     int rows;    // SR
     int halo;    // H
     int steps;   // T
+    int waves;   // NW
 };
 
 struct StripMap {
@@ -45,6 +46,9 @@ inline void strip_tiles(int c, int owned, int halo, int staged, int count, int& 
     last = (c + halo) / owned;
     if (last > count - 1) last = count - 1;
 }
+
+// Wavefront of a tile that stages the cell with index `local`.
+inline int strip_wave(const StripMap& m, int local) { return (local >> 6) / (m.sh.rows / m.sh.waves); }
 
 // Staged index (row * 64 + column) of cell (i, j) in tile (ti, tj).
 inline int strip_local(const StripMap& m, int ti, int tj, int i, int j)

@@ -177,6 +177,42 @@ struct Strip {
     static_assert(OR > 0 && OC > 0 && KR >= R, "strip shape");
 };
 
+// Sources of a wavefront up to which it takes one after the other, with scalar
+// loads (two of 0.15 us a source and step). More are taken by the lanes that hold
+// their cells, each its own ones (two vector loads deep): 40 x 40 sources on 200 x
+// 200, 60 us a step and more otherwise.
+constexpr int kFewPoints = 4;
+
+// The first of the wavefront's entries (in lane order) of this lane or a later one.
+__device__ __forceinline__ int lane_first(const int2* ent, int beg, int end, int lane)
+{
+    while (beg < end) {
+        const int mid = (beg + end) >> 1;
+        if ((ent[mid].x & 63) < lane) beg = mid + 1;
+        else end = mid;
+    }
+    return beg;
+}
+
+// f(row of the strip, point) for the entries [beg, end) of this wavefront on cells
+// of this lane, in input order; own: where lane_first's lies, for more than a few.
+template <int KR, typename F>
+__device__ __forceinline__ void lane_points(const int2* ent, int beg, int end, const int* own, int w, int lane, F f)
+{
+    if (end - beg <= kFewPoints) {
+        for (int x = beg; x < end; ++x) {
+            const int2 e = ent[x];
+            f((e.x & 63) == lane ? (e.x >> 6) - w * KR : -1, e.y);
+        }
+    } else {
+        for (int x = *own; x < end; ++x) {
+            const int2 e = ent[x];
+            if ((e.x & 63) != lane) break;
+            f((e.x >> 6) - w * KR, e.y);
+        }
+    }
+}
+
 // Rows -(R - 1) .. KR + R - 1 (FWD) or -R .. KR + R - 2 of this wavefront's
 // strip of v: the rows of its neighbours through LDS. Two barriers' worth of
 // steps may be in flight, so forward and backward exchanges use separate
@@ -205,7 +241,7 @@ __device__ __forceinline__ void exchange(const float (&v)[KR], float (*first)[DN
 // Forward: nsub (at most T) steps from it0
 // ---------------------------------------------------------------------------
 // One barrier per half step (its first and last rows through LDS) and one more
-// where the tile owns a receiver. A source is added by every tile that stages
+// where the tile owns a receiver. A source is added by every wavefront that stages
 // its cell, a receiver read by the tile that owns it.
 // The arguments are read where they are used: what only the stores or a listed
 // source need is not kept in scalar registers over the steps.
@@ -237,6 +273,7 @@ __device__ __forceinline__ void strip_fwd(StripArgsPtr args, int ti, int tj, int
     __shared__ float h_first[NW][R > 1 ? R - 1 : 1][64], h_last[NW][R][64];
     __shared__ float s_cx[SR][8];  // x-face profiles of the rows: H, then E
     __shared__ float s_ez[SR * 64];
+    __shared__ int s_own[NW][64];  // the lanes' first sources (lane_points)
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int i0 = ti * St::OR - H + w * KR, gj = tj * St::OC - H + lane;  // first row of the strip, column
@@ -317,9 +354,10 @@ __device__ __forceinline__ void strip_fwd(StripArgsPtr args, int ti, int tj, int
     }
     int sbeg = 0, send = 0, rbeg = 0, rend = 0;
     if (args->src.count > 0) {
-        sbeg = args->src.block_off[lt];
-        send = args->src.block_off[lt + 1];
+        sbeg = args->src.block_off[lt * NW + w];
+        send = args->src.block_off[lt * NW + w + 1];
     }
+    if (send - sbeg > kFewPoints) s_own[w][lane] = lane_first(args->src.entries, sbeg, send, lane);
     if (args->rx.count > 0) {
         rbeg = args->rx.off[lt];
         rend = args->rx.off[lt + 1];
@@ -445,15 +483,14 @@ __device__ __forceinline__ void strip_fwd(StripArgsPtr args, int ti, int tj, int
                     pye[q] = cye.re * pye[q] - cye.rf * der[q];
                 }
             }
-            for (int x = sbeg; x < send; ++x) {
+            if (send > sbeg) {
                 const auto& src = again(args)->src;
-                const int2 ent = src.entries[x];
-                const int row = ent.x >> 6;
-                if (row / KR != w) continue;
-                const float scale = src.wave[(long long)ent.y * src.nt + it] * src.dl / src.vol;
+                lane_points<KR>(src.entries, sbeg, send, &s_own[w][lane], w, lane, [&](int row, int point) {
+                    const float scale = src.wave[(long long)point * src.nt + it] * src.dl / src.vol;
 #pragma unroll
-                for (int q = 0; q < KR; ++q)
-                    if (row - w * KR == q && (ent.x & 63) == lane) ez[q] -= cb[q] * scale;
+                    for (int q = 0; q < KR; ++q)
+                        if (row == q) ez[q] -= cb[q] * scale;
+                });
             }
             if (save && it == next) {
                 const auto& hist = again(args)->hist;
@@ -606,6 +643,7 @@ __device__ __forceinline__ void strip_adj(StripAdjArgsPtr args, int ti, int tj, 
     __shared__ float h_first[NW][R > 1 ? R - 1 : 1][64], h_last[NW][R][64];
     __shared__ float s_cx[SR][8];  // x-face profiles of the rows: H, then E
     __shared__ float s_lz[SR * 64];
+    __shared__ int s_own[NW][64];  // the lanes' first sources (lane_points)
     __shared__ float4 s_cy[2][64];  // y-face profiles of the columns: H, then E
     __shared__ float4 s_mat[SR * 64];  // factors of the material terms (a cell's own thread writes and reads them)
     const int lane = threadIdx.x & 63;
@@ -690,26 +728,24 @@ __device__ __forceinline__ void strip_adj(StripAdjArgsPtr args, int ti, int tj, 
     const float invx = args->inv[0], invy = args->inv[1];
     int sbeg = 0, send = 0, rbeg = 0, rend = 0;
     if (args->src.count > 0) {
-        sbeg = args->src.block_off[lt];
-        send = args->src.block_off[lt + 1];
+        sbeg = args->src.block_off[lt * NW + w];
+        send = args->src.block_off[lt * NW + w + 1];
     }
+    if (send - sbeg > kFewPoints) s_own[w][lane] = lane_first(args->src.entries, sbeg, send, lane);
     if (args->rx.count > 0) {
-        rbeg = args->rx.off[lt];
-        rend = args->rx.off[lt + 1];
+        rbeg = args->rx.off[lt * NW + w];
+        rend = args->rx.off[lt * NW + w + 1];
     }
-    // the first 64 receiver cells of the tile: a lane's own one, its data a step ahead
+    // the first 64 receiver cells of the wavefront: a lane's own one, its data a step ahead
     int4 mine = make_int4(-1, 0, 0, 0);
     int first = 0;
     float ahead = 0.0f;
     if (rbeg + lane < rend) {
-        const int4 e = args->rx.grp[rbeg + lane];
-        if ((e.x >> 6) / KR == w) {
-            mine = e;
-            first = args->rx.member[e.y];
-            ahead = args->rx.dgrad[((long long)s * args->rx.nt + it0) * args->rx.nrx + first];
-        }
+        mine = args->rx.grp[rbeg + lane];
+        first = args->rx.member[mine.y];
+        ahead = args->rx.dgrad[((long long)s * args->rx.nt + it0) * args->rx.nrx + first];
     }
-    const bool any_rx = __any(mine.x >= 0) || rend - rbeg > 64;
+    const bool any_rx = rend > rbeg;
 
     // conditions of the strip's rows, one bit each; m_cb and m_cf start with the rows before it
     const unsigned m_in = row_range(i0, KR, 1, g.NX - 2);
@@ -796,7 +832,6 @@ __device__ __forceinline__ void strip_adj(StripAdjArgsPtr args, int ti, int tj, 
             }
             for (int x = rbeg + 64 + lane; x < rend; x += 64) {
                 const int4 e = rx.grp[x];
-                if ((e.x >> 6) / KR != w) continue;
                 float acc = s_lz[e.x];
                 for (int m = 0; m < e.z; ++m) acc += rx.dgrad[at + rx.member[e.y + m]];
                 s_lz[e.x] = acc;
@@ -806,15 +841,14 @@ __device__ __forceinline__ void strip_adj(StripAdjArgsPtr args, int ti, int tj, 
             for (int q = 0; q < KR; ++q) lz[q] = s_lz[(w * KR + q) * 64 + lane];
         }
         // source^T: one value per (step, shot, source), summed over shots later
-        for (int x = sbeg; x < send; ++x) {
+        if (send > sbeg) {
             const auto& a = *again(args);
-            const int2 ent = a.src.entries[x];
-            const int row = ent.x >> 6;
-            if (row / KR != w) continue;
+            lane_points<KR>(a.src.entries, sbeg, send, &s_own[w][lane], w, lane, [&](int row, int point) {
 #pragma unroll
-            for (int q = 0; q < KR; ++q)
-                if (row - w * KR == q && (ent.x & 63) == lane)
-                    a.mg.src_vals[((long long)it * a.g.nshot + s) * a.mg.nsrc + ent.y] = -cb[q] * a.mg.geo * lz[q];
+                for (int q = 0; q < KR; ++q)
+                    if (row == q)
+                        a.mg.src_vals[((long long)it * a.g.nshot + s) * a.mg.nsrc + point] = -cb[q] * a.mg.geo * lz[q];
+            });
         }
         // (electric half step)^T
         {
@@ -1114,7 +1148,7 @@ template <int ORDER, int SIZE>
 StripShape shape_of()
 {
     using P = Shapes<ORDER, SIZE>;
-    return {SIZE, P::KR * P::NW, P::T * (2 * Radius<ORDER>::value - 1), P::T};
+    return {SIZE, P::KR * P::NW, P::T * (2 * Radius<ORDER>::value - 1), P::T, P::NW};
 }
 template <int ORDER, int SIZE>
 void launch_shape(const dim3& grid, const StripArgs& a, hipStream_t st)

@@ -174,3 +174,27 @@ def test_signs_of_zeros_equal_the_one_step_kernels(oracle_built, cuda_device, mo
     for key in ("E", "H", "phi"):
         for k, (a, b) in enumerate(zip(strips[key], steps[key])):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (key, k)
+
+
+@pytest.mark.parametrize("NX,NY,order,nt,nshot", [(45, 70, 2, 26, 1), (45, 70, 4, 9, 2), (61, 209, 2, 9, 14),
+                                                  (50, 90, 2, 8, 48), (50, 90, 4, 5, 40)])
+def test_many_points_match_oracle(oracle_built, cuda_device, monkeypatch, NX, NY, order, nt, nshot):
+    """Sources on a block of cells and along both axes, several on one cell, and receivers on every second cell: more
+    points of a wavefront than it takes one after the other, and more receiver cells than its lanes."""
+    h = oracle_built
+    monkeypatch.delenv("DEEPGPR_AMD_TM2D_TILE_ROWS", raising=False)
+    print(f"[gpu strips] many points {NX}x{NY} o{order} n{nshot}", flush=True)
+    p = _problem(h, (NX, NY, order, nt, nshot, 1, "f32", 2, (5, 4, 6, 7), (0.02, 0.018), False))
+    cells = [(i, j) for i in range(9, 21) for j in range(30, 50)] + [(17, j) for j in range(1, NY - 1, 3)]
+    cells += [(i, 40) for i in range(1, NX - 1, 2)] + [(12, 33)] * 7 + [(30, 60)] * 6
+    rx = [(i, j) for i in range(0, NX - 1) for j in range(i % 2, NY - 1, 2)] + [(12, 34)] * 3
+    rng = np.random.default_rng(7)
+    p.src_loc = np.array([[[(i + s) % (NX - 1), j, 0] for i, j in cells] for s in range(nshot)], np.int32)
+    p.rx_loc = np.array([[[i, j, 0] for i, j in rx] for _ in range(nshot)], np.int32)
+    p.wave = rng.standard_normal((len(cells), nt)).astype(np.float32)
+    p.data_grad = (1e-3 * rng.standard_normal((nshot, nt, len(rx)))).astype(np.float32)
+    cpu = h.run_cpu(p, "oracle")
+    p.storage_type |= TM2D
+    gpu = h.run_gpu(p, api="dgx")
+    bad = h.bitwise_diff(gpu, cpu, h.KEYS_FWD + ("g_src", "g_eps", "g_sig"))
+    assert not bad, bad
