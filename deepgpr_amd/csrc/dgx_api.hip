@@ -1211,7 +1211,10 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
                 }
                 tmp.push_back({blk, s * P->nsource + k, (int)m, k});
             }
-        std::stable_sort(tmp.begin(), tmp.end(), [](const E4& a, const E4& b) { return a.blk < b.blk; });
+        // row sweeps: by cell within a list, the sources of a cell in input order
+        std::stable_sort(tmp.begin(), tmp.end(), [rows](const E4& a, const E4& b) {
+            return a.blk != b.blk ? a.blk < b.blk : rows && a.cell < b.cell;
+        });
         for (const E4& e : tmp) {
             const long long list = xm ? e.blk / g.N[0] : e.blk;  // x-marching: key (list, plane)
             boff[(size_t)list + 1] += 1;

@@ -601,6 +601,12 @@ __device__ __forceinline__ void store_hist_group(void* base, long long idx, fv<V
     }
 }
 
+// Sources of a workgroup up to which every thread looks at each of them. More
+// (they are in order of their cells) a thread searches for its own: with a plane
+// of 80 x 80 sources on 80 x 80 x 80 a workgroup of seven rows looked at 560,
+// 120 us a step more than without them.
+constexpr int kFewSources = 4;
+
 template <int ORDER, int V, bool XY>
 __device__ __forceinline__ void fwd_e_group(const Grid& g, const float* ca, const float* ccurl, const float* cb,
                                             const CF3& Hf, const F3& E, const Cpml& cp, const float* tab, int has_cpml,
@@ -655,8 +661,7 @@ __device__ __forceinline__ void fwd_e_group(const Grid& g, const float* ca, cons
     // again rather than keep them in registers all along
     unsigned m = q.m;
     asm volatile("" : "+v"(m));
-    for (int x = sb; x < se; ++x) {
-        const int2 ent = src.entries[x];
+    auto add = [&](const int2& ent) {
         const unsigned at = (unsigned)ent.x - q.m;
         if (at < (unsigned)V) {
             const fv<V> cbv = ldv<V>(cb, m);
@@ -666,6 +671,21 @@ __device__ __forceinline__ void fwd_e_group(const Grid& g, const float* ca, cons
 #pragma unroll
                 for (int t = 0; t < 3; ++t)
                     if (at == (unsigned)y && t == src.comp) e[t][y] -= cbv[y] * scale;
+        }
+    };
+    if (se - sb <= kFewSources) {
+        for (int x = sb; x < se; ++x) add(src.entries[x]);
+    } else {
+        int x = sb, end = se;  // the first source on the group's cells or beyond them
+        while (x < end) {
+            const int mid = (x + end) >> 1;
+            if ((unsigned)src.entries[mid].x < q.m) x = mid + 1;
+            else end = mid;
+        }
+        for (; x < se; ++x) {
+            const int2 ent = src.entries[x];
+            if ((unsigned)ent.x >= q.m + V) break;
+            add(ent);
         }
     }
     if (hist.active && q.i >= hist.box.x0 && q.i < hist.box.x0 + hist.box.nx && q.j >= hist.box.y0 &&

@@ -103,3 +103,26 @@ def test_faces_close_to_the_middle_match_oracle(oracle_built, cuda_device, shape
     gpu = h.run_gpu(p, api="dgx")
     bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
     assert not bad, bad
+
+
+@pytest.mark.parametrize("NZ,order,comp,nshot", [(66, 4, 1, 1), (71, 2, 2, 2), (68, 4, 0, 1)])
+def test_many_sources_match_oracle(oracle_built, cuda_device, NZ, order, comp, nshot):
+    """Sources on whole planes, in no order, several on one cell: more of a workgroup than every thread looks at."""
+    h = oracle_built
+    print(f"[gpu row sweeps] many sources {NZ} {order} {comp}", flush=True)
+    p = h.make_problem(56, 54, NZ, order=order, nt=5, nshot=nshot, nsrc=1, nrx=5, seed=37, pml=(4, 3, 5, 4, 4, 6),
+                       d=(0.02, 0.017, 0.015))
+    cells = [(20, j, k) for j in range(0, 53, 2) for k in range(0, NZ - 1)] + [(i, 30, 33) for i in range(55)]
+    cells += [(20, 16, 9)] * 7 + [(5, 5, NZ - 2)] * 3
+    rng = np.random.default_rng(5)
+    order_ = rng.permutation(len(cells))
+    p.src_loc = np.array([[list(cells[k]) for k in order_] for _ in range(nshot)], np.int32)
+    p.wave = rng.standard_normal((len(cells), 5)).astype(np.float32)
+    p.src_comp = p.rx_comp = comp
+    for s in range(nshot):
+        for r in range(5):
+            p.rx_loc[s, r] = [18 + r, 16, 8 + r]
+    cpu = h.run_cpu(p, "oracle")
+    gpu = h.run_gpu(p, api="dgx")
+    bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
+    assert not bad, bad
