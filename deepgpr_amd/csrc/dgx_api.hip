@@ -549,7 +549,7 @@ bool xmarch3d()
 // (dgx_rows.hip); DEEPGPR_AMD_3D_SWEEP=cells keeps the one-thread-per-cell
 // sweeps, which order 8, smaller 3D grids and the general 2D path take (same
 // bits). So do the switches of those sweeps. Read at every solve.
-bool row_sweeps(const Grid& g, int order)
+bool row_sweeps(const Grid& g, int order, bool backward)
 {
     const char* v = std::getenv("DEEPGPR_AMD_3D_SWEEP");
     if (v && (std::strcmp(v, "cells") == 0 || std::strcmp(v, "xmarch") == 0)) return false;
@@ -557,7 +557,7 @@ bool row_sweeps(const Grid& g, int order)
     if (v && std::strcmp(v, "off") == 0) return false;
     v = std::getenv("DEEPGPR_AMD_3D_INTERLEAVE");
     if (v && std::strcmp(v, "off") == 0) return false;
-    return adj3d_fused() && row_sweep_applies(g.N, g.pml, order);
+    return adj3d_fused() && row_sweep_applies(g.N, g.pml, order, backward);
 }
 
 // Static rule for the tile rows of a single fused TM solve. Small solves
@@ -1163,7 +1163,7 @@ int run_forward(const dgx_solve* P, hipStream_t stream, void* fixed = nullptr, s
     const bool fused = tm && tm2d_fused();
     const bool xm = !fixed && !tm && xmarch3d();
     const XmTiles xt = xm_tiles(g, pl.order);
-    const bool rows = !fixed && !tm && !xm && row_sweeps(g, pl.order);
+    const bool rows = !fixed && !tm && !xm && row_sweeps(g, pl.order, false);
     const RowMap rm = rows ? row_map(g, pl.order) : RowMap{};
     if (fixed && pl.kind == kInt8 && pl.history) {
         set_error("dgx_forward_noalloc: INT8 histories need a scratch frame; use dgx_forward");
@@ -1662,7 +1662,7 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
 
     const bool xm = !tm && xmarch3d();
     const XmTiles xt = xm_tiles(g, pl.order);
-    const bool rows = !tm && !xm && row_sweeps(g, pl.order);
+    const bool rows = !tm && !xm && row_sweeps(g, pl.order, true);
     const RowMap rm = rows ? row_map(g, pl.order) : RowMap{};
     const bool fuse3 = !tm && !xm && !rows && adj3d_fused();
 
@@ -2824,7 +2824,7 @@ DGX_API long long dgx_scratch_bytes(const dgx_solve* solve, int backward)
         if (xmarch3d()) {
             const XmTiles xt = xm_tiles(g, pl.order);
             bytes += ((long long)xt.nty * xt.ntz * g.nshot + 1) * 4;
-        } else if (row_sweeps(g, pl.order)) {
+        } else if (row_sweeps(g, pl.order, false)) {
             // source and receiver lists
             bytes += 2 * ((long long)row_map(g, pl.order).total * g.nshot + 1) * 4;
         } else {
@@ -2838,7 +2838,7 @@ DGX_API long long dgx_scratch_bytes(const dgx_solve* solve, int backward)
         // adjoint channel weights of the general (non-2D-TM) path
         const bool tm_shape = (solve->storage_type & kFlagTm2d) && g.N[2] == 2 && solve->source_component == 2 &&
                               pl.kind != kInt8;
-        if (!tm_shape && !xmarch3d() && !row_sweeps(g, pl.order)) bytes += (adj3d_fused() ? 48LL : 24LL) * g.nshot * g.cells;
+        if (!tm_shape && !xmarch3d() && !row_sweeps(g, pl.order, true)) bytes += (adj3d_fused() ? 48LL : 24LL) * g.nshot * g.cells;
     }
     return bytes;
 }

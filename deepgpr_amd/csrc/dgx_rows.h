@@ -76,18 +76,32 @@ inline bool row_face_fits(int n, int p, bool high)
 // order-8 cell has so many taps that its values fill the registers of a
 // thread (us per step on an MI355X, row sweeps / one thread per cell: forward
 // 118 / 100, adjoint 199 / 152 on 138 x 120 x 152 fields).
-inline bool row_sweep_applies(const int N[3], const int pml[6], int order)
+//
+// Rows of more than 512 cells need workgroups of 5 to 8 wavefronts, a row or two
+// each, and fewer of those share a compute unit. Forward and adjoint, us a step,
+// rows / one thread per cell, fields of 111 x 111 (CPML 10: 62 % of the rows
+// plain), 151 x 151 (CPML 30: 31 %) and 61 x 61 (CPML 10: 39 %) rows:
+//   order 4   501 cells   172 / 181   217 / 304    389 / 575   534 / 840     63 /  79    85 / 117
+//   order 4   521         241 / 189   326 / 318    562 / 596   831 / 860     90 /  80   137 / 120
+//   order 4   701         293 / 249   378 / 414    648 / 762   912 / 1078    99 / 101   146 / 163
+//   order 2   521         177 / 165   225 / 259    395 / 550   568 / 792     66 /  74    92 / 110
+//   order 2   701         220 / 215   278 / 342    475 / 702   682 / 988     76 /  93   112 / 145
+// Hence: order 4 from 704 cells again, and a forward sweep only where fewer than
+// half of the rows are plain.
+inline bool row_sweep_applies(const int N[3], const int pml[6], int order, bool backward = true)
 {
     if (order > 4) return false;
-    long long cells = 1;
+    long long cells = 1, rows = 1;
     for (int a = 0; a < 3; ++a) {
         int lo, hi;
         row_plain_range(N[a], pml[2 * a], pml[2 * a + 1], 4, lo, hi);
         if (hi < lo) return false;
         if (a == 2 && hi - lo + 1 < 32) return false;
+        if (a == 2) rows = cells;
         cells *= hi - lo + 1;
         if (!row_face_fits(N[a], pml[2 * a], false) || !row_face_fits(N[a], pml[2 * a + 1], true)) return false;
     }
+    if (N[2] > 512 && ((order == 4 && N[2] < 704) || (!backward && 2 * rows >= 1LL * N[0] * N[1]))) return false;
     return cells >= 65536 && N[2] <= 1024 && 1LL * N[0] * N[1] * N[2] < (1LL << 30);
 }
 
@@ -132,8 +146,12 @@ inline RowMap make_row_map(const int N[3], const int pml[6], int R, int V, int m
     row_plain_range(N[0], pml[0], pml[1], R, m.xlo, m.xhi);
     row_plain_range(N[1], pml[2], pml[3], R, m.ylo, m.yhi);
     row_plain_range(N[2], pml[4], pml[5], R, m.zlo, m.zhi);
-    m.plain = make_row_kind(N[2], V, max_threads);
+    // A long row takes more than max_threads threads in edge groups, and the launch
+    // has as many for every workgroup: the plain ones then hold rows for all of
+    // them (two rows of 561 cells in 282 threads of 320, not one in 141).
     m.edge = make_row_kind(N[2], V / 2, max_threads);
+    const int most = (m.edge.rb * m.edge.gpr + 63) / 64 * 64;
+    m.plain = make_row_kind(N[2], V, most > max_threads ? most : max_threads);
     set_row_ends(m.plain, V, m.zlo, m.zhi);
     set_row_ends(m.edge, V / 2, m.zlo, m.zhi);
     const int tp = m.plain.rb * m.plain.gpr, te = m.edge.rb * m.edge.gpr;

@@ -126,3 +126,18 @@ def test_many_sources_match_oracle(oracle_built, cuda_device, NZ, order, comp, n
     gpu = h.run_gpu(p, api="dgx")
     bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
     assert not bad, bad
+
+
+@pytest.mark.parametrize("shape,order,pml", [((48, 46, 707), 4, (6, 5, 7, 4, 5, 9)), ((48, 46, 541), 2, (6, 5, 7, 4, 5, 9)),
+                                             ((30, 33, 1022), 4, (4, 4, 4, 4, 6, 6))])
+def test_long_rows_match_oracle(oracle_built, cuda_device, shape, order, pml):
+    """Rows that need workgroups of more than 256 threads."""
+    h = oracle_built
+    print(f"[gpu row sweeps] long rows {shape} {order}", flush=True)
+    p = h.make_problem(*shape, order=order, nt=5, nshot=1, nsrc=2, nrx=4, seed=53, pml=pml, d=(0.02, 0.017, 0.015))
+    p.src_loc[0, 0] = [shape[0] // 2, shape[1] // 2, shape[2] // 2]
+    p.rx_loc[0, 0] = [shape[0] // 2, 1 + shape[1] // 2, shape[2] - 3]
+    cpu = h.run_cpu(p, "oracle")
+    gpu = h.run_gpu(p, api="dgx")
+    bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
+    assert not bad, bad
