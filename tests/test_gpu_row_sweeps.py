@@ -141,3 +141,20 @@ def test_long_rows_match_oracle(oracle_built, cuda_device, shape, order, pml):
     gpu = h.run_gpu(p, api="dgx")
     bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
     assert not bad, bad
+
+
+@pytest.mark.parametrize("NZ,order", [(261, 4), (327, 2)])
+def test_receivers_on_whole_rows_match_oracle(oracle_built, cuda_device, NZ, order):
+    """More receivers on the rows of a workgroup than its live wavefronts have threads; some of its wavefronts idle."""
+    h = oracle_built
+    print(f"[gpu row sweeps] receivers on whole rows {NZ} {order}", flush=True)
+    rows = [(1, 20), (20, 20), (20, 21), (20, 22), (21, 1), (41, 40)]
+    cells = [(i, j, k) for i, j in rows for k in range(NZ)] + [(20, 20, 33)] * 3
+    p = h.make_problem(44, 42, NZ, order=order, nt=4, nshot=1, nsrc=1, nrx=len(cells), seed=59, pml=(4, 3, 4, 5, 6, 4),
+                       d=(0.02, 0.017, 0.015))
+    p.src_loc[0, 0] = [20, 21, 40]
+    p.rx_loc = np.array([cells], np.int32)
+    cpu = h.run_cpu(p, "oracle")
+    gpu = h.run_gpu(p, api="dgx")
+    bad = h.bitwise_diff(gpu, cpu, list(h.KEYS_FWD) + list(h.KEYS_BWD))
+    assert not bad, bad
