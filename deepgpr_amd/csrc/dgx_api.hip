@@ -1061,21 +1061,14 @@ void row_receiver_lists(const Grid& g, const RowMap& rm, const std::vector<int>&
 {
     const long long per = rm.total;
     std::vector<std::pair<long long, int2>> tmp;
+    tmp.reserve((size_t)g.nshot * nrx);
     for (int s = 0; s < g.nshot; ++s)
         for (int r = 0; r < nrx; ++r) {
             const int* L = &rloc[((size_t)s * nrx + r) * 3];
             tmp.push_back({row_block_of(rm, L[0], L[1]) + per * s,
                            make_int2((int)(L[0] * g.st0 + (long long)L[1] * g.N[2] + L[2]), r)});
         }
-    std::stable_sort(tmp.begin(), tmp.end(), [](const std::pair<long long, int2>& x,
-                                                const std::pair<long long, int2>& y) { return x.first < y.first; });
-    off.assign((size_t)(per * g.nshot) + 1, 0);
-    ent.clear();
-    for (const auto& e : tmp) {
-        off[(size_t)e.first + 1] += 1;
-        ent.push_back(e.second);
-    }
-    for (size_t k = 1; k < off.size(); ++k) off[k] += off[k - 1];
+    group_lists(tmp, per * g.nshot, off, ent);
 }
 
 // The receiver groups (receiver_groups) of the row sweeps by owning workgroup.
@@ -1084,20 +1077,13 @@ void row_receiver_groups(const Grid& g, const RowMap& rm, const std::vector<int>
 {
     const long long per = rm.total;
     std::vector<std::pair<long long, int4>> tmp;
+    tmp.reserve(gshot.size());
     for (size_t q = 0; q < gshot.size(); ++q) {
         const int i = (int)(gcell[q] / g.st0), j = (int)(gcell[q] % g.st0) / g.N[2];
         tmp.push_back({row_block_of(rm, i, j) + per * gshot[q],
                        make_int4((int)gcell[q], goff[q], goff[q + 1] - goff[q], 0)});
     }
-    std::stable_sort(tmp.begin(), tmp.end(), [](const std::pair<long long, int4>& x,
-                                                const std::pair<long long, int4>& y) { return x.first < y.first; });
-    off.assign((size_t)(per * g.nshot) + 1, 0);
-    grp.clear();
-    for (const auto& e : tmp) {
-        off[(size_t)e.first + 1] += 1;
-        grp.push_back(e.second);
-    }
-    for (size_t k = 1; k < off.size(); ++k) off[k] += off[k - 1];
+    group_lists(tmp, per * g.nshot, off, grp);
 }
 
 // Device copy of a host-built list (nothing to do for an empty one).
