@@ -122,14 +122,16 @@ def model_bytes_per_cell(w, args):
     return fwd, adj
 
 
-def kernel_bytes(kernel: str, w, args, steps: float = 1.0) -> float:
+def kernel_bytes(kernel: str, w, args, steps: float = 1.0, ran=()) -> float:
     """Algorithmic bytes of ONE launch of a kernel (one time step, all shots of
     one call; `steps` time steps for the strip kernels, which read and write
-    the state once a launch and the Ez history once a step). The one-step 2D TM
-    kernels carry the per-cell model above times the cells they advance; the
-    gradient accumulators belong to the reduction kernel while it is separate.
-    The split kernels carry their own share of
-    the compulsory loads/stores."""
+    the state once a launch and the Ez history once a step, and for the sum of
+    their material terms). The one-step 2D TM kernels carry the per-cell model
+    above times the cells they advance; the gradient accumulators belong to the
+    reduction kernel while it is separate. The split kernels carry their own
+    share of the compulsory loads/stores. `ran`: the kernels of the same run,
+    which tell the row sweeps (no stored channel weights) from the
+    one-thread-per-cell sweeps under the same names."""
     shots = args.shots_per_call or w.source_location.shape[0]
     ext = w.extended_cells()
     cells = ext * shots
@@ -145,13 +147,26 @@ def kernel_bytes(kernel: str, w, args, steps: float = 1.0) -> float:
     if kernel == "tm_step_adj":
         return (adj - acc_b) * cells
     if kernel == "tm_grad_reduce":
-        return acc_b * w.sampling_interval * ext  # one launch per saved step, accumulators of all shots
+        # accumulators of all shots read and written once, two terms of each shot a saved step
+        saves = steps / w.sampling_interval if "tm_strip_adj" in ran else 1.0
+        return acc_b * w.sampling_interval * ext + saves * 2 * 4 * cells
     if kernel == "fwd_h":
         core = 24 if two_d else 40      # E read, H read+write, ch_curl
         return cells * core + 8 * ph
     if kernel == "fwd_e":
         core = 24 if two_d else 48      # H read, E read+write, ca, ce_curl (+ce_rhs in 3D)
         return cells * (core + comps * hist_b * frames / w.sampling_interval) + 8 * pe
+    if kernel in ("adj_weights_e", "adj_weights_h"):
+        # lambda (3) + curl coefficient read, six channel weights written, lambda psi read+write
+        return cells * 40 + 8 * (pe if kernel == "adj_weights_e" else ph)
+    if kernel == "adj_e_w":
+        # gather_e, then the H-side weights: W_E read, lambda_H read+write, hcurl, W_H written
+        return cells * 76 + 8 * ph
+    if "adj_weights_e" in ran:  # gathers of stored weights
+        if kernel == "adj_e":
+            return cells * 48           # six channel weights read, lambda_H read+write
+        if kernel == "adj_h":
+            return cells * 52           # six channel weights read, lambda_E read+write, ca
     if kernel == "adj_e":
         return cells * 40 + 8 * pe      # lambda_E, ccurl read, lambda_H read+write, lambda psi_E read+write
     if kernel == "adj_h":
@@ -359,14 +374,16 @@ def main():
             if cnt.value:
                 kernels[name.decode()] = (tot.value, cnt.value)
         lib.dgx_set_kernel_timing(0)
-        ranked = sorted(((t, n) for n, (t, c) in kernels.items() if kernel_bytes(n, w, args) > 0), reverse=True)
+        ranked = sorted(((t, n) for n, (t, c) in kernels.items() if kernel_bytes(n, w, args, ran=kernels) > 0),
+                        reverse=True)
         if ranked:
             _, dom = ranked[0]
             tot, cnt = kernels[dom]
             avg_s = tot / cnt / 1e3
-            bytes_launch = kernel_bytes(dom, w, args, w.nt / cnt)
+            bytes_launch = kernel_bytes(dom, w, args, w.nt / cnt, kernels)
             achieved = bytes_launch / avg_s / 1e9
-            measured = MEASURED_TRAFFIC.get((args.workload, dom, args.storage, args.accumulator, chunk))
+            measured = None if "adj_weights_e" in kernels else MEASURED_TRAFFIC.get(
+                (args.workload, dom, args.storage, args.accumulator, chunk))
             roofline = {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                         "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                         "traffic": int(measured[0]) if measured else None,
