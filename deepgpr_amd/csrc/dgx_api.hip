@@ -1552,6 +1552,26 @@ MatGrad mat_step(const Plan& pl, const dgx_solve* P, MatGrad mg, int it, int nt,
     return mg;
 }
 
+// Per-shot material terms of one saved step of a 2D TM adjoint, in floats.
+long long material_terms_len(const Plan& pl) { return 2 * (long long)pl.g.nshot * pl.box.cells; }
+
+// Saved steps whose terms a 2D TM adjoint holds. Two for the one-step kernels: a
+// launch writes one while it sums the other (the previous saved step). The strip
+// kernels of one shot sum in registers. Those of several shots hold more before
+// the sum kernel adds them: a sum of few cells is a launch and its latency, whose
+// cost the steps share (5 shots of 342 x 264, 400 steps, a gradient: 11.1 ms with
+// a sum after each launch, 9.7 now). Their buffers take no more than two did, or
+// 32 MiB: 20 shots of 441 x 241 keep two steps, whose sum is bound by its bytes. A
+// sum of more than 32 steps would be a longer chain and no fewer bytes.
+// dgx_scratch_bytes counts them by the same rule.
+int held_saves(const Plan& pl, bool strips)
+{
+    if (!strips) return 2;
+    if (pl.g.nshot == 1) return 0;
+    const long long fit = (8LL << 20) / std::max(material_terms_len(pl), 1LL);
+    return (int)std::max<long long>(2, std::min<long long>({32, pl.nt_saved, fit}));
+}
+
 int run_backward(const dgx_solve* P, hipStream_t stream)
 {
     CallStream call(stream);
@@ -1713,20 +1733,9 @@ int run_backward(const dgx_solve* P, hipStream_t stream)
         tgrad.src_vals = (float*)d_svals.p;
         tgrad.nsrc = P->nsource;
     }
-    // Two buffers: a launch writes one while it sums the other (the previous
-    // saved step). The strip kernels hold up to strip_saves saved steps of
-    // several shots before the sum kernel adds them: a sum of few cells is a
-    // launch and its latency, whose cost the steps share (5 shots of 342 x 264,
-    // 400 steps, a gradient: 11.1 ms with a sum after each launch, 9.7 now).
-    // Their buffers take no more than two did, or 32 MiB: 20 shots of 441 x 241
-    // keep two steps, whose sum is bound by its bytes. A sum of more than 32
-    // steps would be a longer chain and no fewer bytes.
-    const long long terms_len = 2 * (long long)g.nshot * pl.box.cells;
-    int strip_saves = 2;
-    if (strips)
-        strip_saves = (int)std::min<long long>(32, std::max<long long>(2, (8LL << 20) / std::max(terms_len, 1LL)));
-    if (fused && want_mat && !(strips && g.nshot == 1) &&
-        !d_terms.alloc((size_t)strip_saves * terms_len * sizeof(float))) {
+    const long long terms_len = material_terms_len(pl);
+    int strip_saves = held_saves(pl, strips);
+    if (fused && want_mat && strip_saves > 0 && !d_terms.alloc((size_t)strip_saves * terms_len * sizeof(float))) {
         (void)hipGetLastError();  // out of memory: two may still fit
         strip_saves = 2;
         if (!d_terms.alloc((size_t)strip_saves * terms_len * sizeof(float))) {
@@ -2811,8 +2820,9 @@ DGX_API long long dgx_scratch_bytes(const dgx_solve* solve, int backward)
             const XmTiles xt = xm_tiles(g, pl.order);
             bytes += ((long long)xt.nty * xt.ntz * g.nshot + 1) * 4;
         } else if (row_sweeps(g, pl.order, false)) {
-            // source and receiver lists
+            // source and receiver lists, CPML profiles by cell
             bytes += 2 * ((long long)row_map(g, pl.order).total * g.nshot + 1) * 4;
+            if (pl.has_cpml) bytes += 8LL * (g.N[0] + g.N[1] + g.N[2]) * 4;
         } else {
             bytes += (cell_sweep(g, pl.order).blocks + 1) * 4;
         }
@@ -2824,6 +2834,9 @@ DGX_API long long dgx_scratch_bytes(const dgx_solve* solve, int backward)
         // adjoint channel weights of the general (non-2D-TM) path
         const bool tm_shape = (solve->storage_type & kFlagTm2d) && g.N[2] == 2 && solve->source_component == 2 &&
                               pl.kind != kInt8;
+        if (tm_shape && tm2d_fused() && (solve->eps_r_requires_grad || solve->sigma_requires_grad))
+            bytes += 4 * material_terms_len(pl) *
+                     held_saves(pl, tm2d_strips() && strip_applies(pl.order, tm_grid_of(pl, kTmBI)));
         if (!tm_shape && !xmarch3d() && !row_sweeps(g, pl.order, true)) bytes += (adj3d_fused() ? 48LL : 24LL) * g.nshot * g.cells;
     }
     return bytes;

@@ -148,7 +148,11 @@ DGX_API int dgx_model_checks(const float* er, const float* se, const float* mr, 
 DGX_API int dgx_codec_roundtrip(const float* input, void* encoded, float* decoded, long long count,
                                 int storage_kind, int conversion_backend, dgx_stream_t stream);
 /* Device memory a solve needs beyond the caller's arrays (bytes), for
- * admission by HBM footprint. No counterpart in the reference. */
+ * admission by HBM footprint. No counterpart in the reference. Counted are the
+ * terms that grow with the grid or the history: FP64 accumulators, CPML copies,
+ * channel weights, INT8 scratch frames, the per-shot gradient terms that 2D
+ * adjoints hold between their sums; not the compact copy of a 2D state (less
+ * than the caller's fields). */
 DGX_API long long dgx_scratch_bytes(const dgx_solve* solve, int backward);
 
 /* Per-launch kernel timing with HIP events on the launch stream, for
