@@ -178,9 +178,11 @@ struct Strip {
 };
 
 // Sources of a wavefront up to which it takes one after the other, with scalar
-// loads (two of 0.15 us a source and step). More are taken by the lanes that hold
-// their cells, each its own ones (two vector loads deep): 40 x 40 sources on 200 x
-// 200, 60 us a step and more otherwise.
+// loads (0.3 us a source and step). More are taken by the lanes that hold their
+// cells, each finding its own by bisection: 20 x 20 sources on 200 x 200 (order 2,
+// forward), 75 us a step one after the other, 7 this way. The branches that points
+// need are laid out of the way of the other wavefronts (adjoint of 441 x 241 x 20
+// shots, two steps: 70.6 and 69.0 us).
 constexpr int kFewPoints = 4;
 
 // The first of the wavefront's entries (in lane order) of this lane or a later one.
@@ -195,9 +197,9 @@ __device__ __forceinline__ int lane_first(const int2* ent, int beg, int end, int
 }
 
 // f(row of the strip, point) for the entries [beg, end) of this wavefront on cells
-// of this lane, in input order; own: where lane_first's lies, for more than a few.
+// of this lane, in input order.
 template <int KR, typename F>
-__device__ __forceinline__ void lane_points(const int2* ent, int beg, int end, const int* own, int w, int lane, F f)
+__device__ __forceinline__ void lane_points(const int2* ent, int beg, int end, int w, int lane, F f)
 {
     if (end - beg <= kFewPoints) {
         for (int x = beg; x < end; ++x) {
@@ -205,7 +207,7 @@ __device__ __forceinline__ void lane_points(const int2* ent, int beg, int end, c
             f((e.x & 63) == lane ? (e.x >> 6) - w * KR : -1, e.y);
         }
     } else {
-        for (int x = *own; x < end; ++x) {
+        for (int x = lane_first(ent, beg, end, lane); x < end; ++x) {
             const int2 e = ent[x];
             if ((e.x & 63) != lane) break;
             f((e.x >> 6) - w * KR, e.y);
@@ -273,7 +275,6 @@ __device__ __forceinline__ void strip_fwd(StripArgsPtr args, int ti, int tj, int
     __shared__ float h_first[NW][R > 1 ? R - 1 : 1][64], h_last[NW][R][64];
     __shared__ float s_cx[SR][8];  // x-face profiles of the rows: H, then E
     __shared__ float s_ez[SR * 64];
-    __shared__ int s_own[NW][64];  // the lanes' first sources (lane_points)
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int i0 = ti * St::OR - H + w * KR, gj = tj * St::OC - H + lane;  // first row of the strip, column
@@ -357,7 +358,6 @@ __device__ __forceinline__ void strip_fwd(StripArgsPtr args, int ti, int tj, int
         sbeg = args->src.block_off[lt * NW + w];
         send = args->src.block_off[lt * NW + w + 1];
     }
-    if (send - sbeg > kFewPoints) s_own[w][lane] = lane_first(args->src.entries, sbeg, send, lane);
     if (args->rx.count > 0) {
         rbeg = args->rx.off[lt];
         rend = args->rx.off[lt + 1];
@@ -483,9 +483,9 @@ __device__ __forceinline__ void strip_fwd(StripArgsPtr args, int ti, int tj, int
                     pye[q] = cye.re * pye[q] - cye.rf * der[q];
                 }
             }
-            if (send > sbeg) {
+            if (__builtin_expect(send > sbeg, 0)) {
                 const auto& src = again(args)->src;
-                lane_points<KR>(src.entries, sbeg, send, &s_own[w][lane], w, lane, [&](int row, int point) {
+                lane_points<KR>(src.entries, sbeg, send, w, lane, [&](int row, int point) {
                     const float scale = src.wave[(long long)point * src.nt + it] * src.dl / src.vol;
 #pragma unroll
                     for (int q = 0; q < KR; ++q)
@@ -643,7 +643,6 @@ __device__ __forceinline__ void strip_adj(StripAdjArgsPtr args, int ti, int tj, 
     __shared__ float h_first[NW][R > 1 ? R - 1 : 1][64], h_last[NW][R][64];
     __shared__ float s_cx[SR][8];  // x-face profiles of the rows: H, then E
     __shared__ float s_lz[SR * 64];
-    __shared__ int s_own[NW][64];  // the lanes' first sources (lane_points)
     __shared__ float4 s_cy[2][64];  // y-face profiles of the columns: H, then E
     __shared__ float4 s_mat[SR * 64];  // factors of the material terms (a cell's own thread writes and reads them)
     const int lane = threadIdx.x & 63;
@@ -731,7 +730,6 @@ __device__ __forceinline__ void strip_adj(StripAdjArgsPtr args, int ti, int tj, 
         sbeg = args->src.block_off[lt * NW + w];
         send = args->src.block_off[lt * NW + w + 1];
     }
-    if (send - sbeg > kFewPoints) s_own[w][lane] = lane_first(args->src.entries, sbeg, send, lane);
     if (args->rx.count > 0) {
         rbeg = args->rx.off[lt * NW + w];
         rend = args->rx.off[lt * NW + w + 1];
@@ -818,7 +816,7 @@ __device__ __forceinline__ void strip_adj(StripAdjArgsPtr args, int ti, int tj, 
             });
         }
         // receivers^T
-        if (any_rx) {
+        if (__builtin_expect(any_rx, 0)) {
             const auto& rx = again(args)->rx;
 #pragma unroll
             for (int q = 0; q < KR; ++q) s_lz[(w * KR + q) * 64 + lane] = lz[q];
@@ -841,9 +839,9 @@ __device__ __forceinline__ void strip_adj(StripAdjArgsPtr args, int ti, int tj, 
             for (int q = 0; q < KR; ++q) lz[q] = s_lz[(w * KR + q) * 64 + lane];
         }
         // source^T: one value per (step, shot, source), summed over shots later
-        if (send > sbeg) {
+        if (__builtin_expect(send > sbeg, 0)) {
             const auto& a = *again(args);
-            lane_points<KR>(a.src.entries, sbeg, send, &s_own[w][lane], w, lane, [&](int row, int point) {
+            lane_points<KR>(a.src.entries, sbeg, send, w, lane, [&](int row, int point) {
 #pragma unroll
                 for (int q = 0; q < KR; ++q)
                     if (row == q)
