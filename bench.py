@@ -186,9 +186,9 @@ def kernel_bytes(kernel: str, w, args, steps: float = 1.0, ran=()) -> float:
 # accumulator, shots per call): traffic depends on all of them. The commands
 # and per-kernel tables are in the profiles/*.md file named with each entry.
 MEASURED_TRAFFIC = {
-    ("c3", "adj_e", "float32", "float64", 1): (1334.7e6, "profiles/c3_layered_3d_o4_kernels.md"),
-    ("c2", "tm_strip_adj", "float32", "float64", 20): (249.2e6, "profiles/c2_fwi_2d_o4_strip_kernels.md"),
-    ("c2", "tm_strip_fwd", "float32", "float64", 20): (162.1e6, "profiles/c2_fwi_2d_o4_strip_kernels.md"),
+    ("c3", "adj_e", "float32", "float64", 1): (1329.7e6, "profiles/c3_layered_3d_o4_kernels.md"),
+    ("c2", "tm_strip_adj", "float32", "float64", 20): (248.8e6, "profiles/c2_fwi_2d_o4_strip_kernels.md"),
+    ("c2", "tm_strip_fwd", "float32", "float64", 20): (162.5e6, "profiles/c2_fwi_2d_o4_strip_kernels.md"),
 }
 
 
