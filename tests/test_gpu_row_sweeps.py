@@ -129,9 +129,10 @@ def test_many_sources_match_oracle(oracle_built, cuda_device, NZ, order, comp, n
 
 
 @pytest.mark.parametrize("shape,order,pml", [((48, 46, 707), 4, (6, 5, 7, 4, 5, 9)), ((48, 46, 541), 2, (6, 5, 7, 4, 5, 9)),
-                                             ((30, 33, 1022), 4, (4, 4, 4, 4, 6, 6))])
+                                             ((30, 33, 1022), 4, (4, 4, 4, 4, 6, 6)),
+                                             ((60, 58, 541), 2, (3, 3, 2, 3, 5, 9)), ((56, 58, 706), 4, (3, 0, 2, 3, 5, 9))])
 def test_long_rows_match_oracle(oracle_built, cuda_device, shape, order, pml):
-    """Rows that need workgroups of more than 256 threads."""
+    """Rows that need workgroups of more than 256 threads; on the last two grids in the adjoint alone."""
     h = oracle_built
     print(f"[gpu row sweeps] long rows {shape} {order}", flush=True)
     p = h.make_problem(*shape, order=order, nt=5, nshot=1, nsrc=2, nrx=4, seed=53, pml=pml, d=(0.02, 0.017, 0.015))
